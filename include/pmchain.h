@@ -457,6 +457,14 @@ pm_status pm_project_mass(const float* pos_a, const float* pos_b, const float* m
                           int64_t n_particles, float lo_a, float lo_b, float binw_a,
                           float binw_b, int32_t bins, float* img, void* scratch,
                           hipStream_t stream);
+/* The same image bit for bit with workspace for the particles too (work:
+ * pm_project_work_bytes(n, bins) bytes of device memory, 8-byte aligned): large sets are
+ * partitioned by image tile and summed in LDS instead of by global atomics. */
+pm_status pm_project_work_bytes(int64_t n_particles, int32_t bins, int64_t* out);
+pm_status pm_project_mass_work(const float* pos_a, const float* pos_b, const float* mass,
+                               int64_t n_particles, float lo_a, float lo_b, float binw_a,
+                               float binw_b, int32_t bins, float* img, void* work,
+                               hipStream_t stream);
 
 /* dst = src (count floats): a plain streaming copy of known size, used to calibrate
  * profiler byte counters (no reference counterpart). */
