@@ -22,6 +22,7 @@
 
 #include <cstdio>
 
+#include "pm_mg_tile.h"
 #include "pm_reduce.h"
 #include "pm_timing.h"
 #include "pm_warm.h"
@@ -1713,12 +1714,58 @@ pm_status bottom(pm_mg* mg, size_t l, hipStream_t s) {
   return PM_OK;
 }
 
+// MIXED levels below the finest and up to this size run each leg in one launch when it has one
+// or two sweeps (pm_mg_tile.h, with the measurements behind the line). On PLAIN's halving
+// levels the V(2,2) legs measured no gain (a 128^3 step 1618 us per 4 steps without, 1629
+// with): they keep a launch per pass.
+constexpr int kLegMax = 72;
+
+bool use_legs(const pm_mg* mg, size_t l) {
+  const Level& L = mg->lv[l];
+  auto few = [](int sweeps) { return sweeps == 1 || sweeps == 2; };
+  return mg->use_small_sweep && mg->d.mode == PM_MG_MIXED && l > 0 && L.tmp && L.n <= kLegMax &&
+         few(mg->d.pre_sweeps) && few(mg->d.post_sweeps);
+}
+
+pm_status leg_down(const Level& L, const Level& C, int sweeps, hipStream_t s) {
+  const int nb = pm::tile::blocks_per_axis(L.n);
+  const unsigned grid = static_cast<unsigned>(nb) * nb * nb;
+  PM_TIMED(level_name("mg.leg_down", L.n), 9.0 * L.nodes(), s);
+  if (sweeps == 1)
+    pm::tile::down_kernel<1><<<grid, pm::tile::T, 0, s>>>(L.rhs, L.tmp, C.rhs, C.phi, L.n, C.n, nb,
+                                                         L.h2, L.inv_h2);
+  else
+    pm::tile::down_kernel<2><<<grid, pm::tile::T, 0, s>>>(L.rhs, L.tmp, C.rhs, C.phi, L.n, C.n, nb,
+                                                         L.h2, L.inv_h2);
+  PM_CHECK_LAUNCH("down_kernel");
+  return PM_OK;
+}
+
+pm_status leg_up(const Level& L, const Level& C, int sweeps, hipStream_t s) {
+  const int nb = pm::tile::blocks_per_axis(L.n);
+  const unsigned grid = static_cast<unsigned>(nb) * nb * nb;
+  PM_TIMED(level_name("mg.leg_up", L.n), 12.5 * L.nodes(), s);
+  if (sweeps == 1)
+    pm::tile::up_kernel<1><<<grid, pm::tile::T, 0, s>>>(L.tmp, L.rhs, C.phi, L.phi, L.n, C.n, nb,
+                                                       L.h2);
+  else
+    pm::tile::up_kernel<2><<<grid, pm::tile::T, 0, s>>>(L.tmp, L.rhs, C.phi, L.phi, L.n, C.n, nb,
+                                                       L.h2);
+  PM_CHECK_LAUNCH("up_kernel");
+  return PM_OK;
+}
+
 pm_status vcycle(pm_mg* mg, size_t l, hipStream_t s) {
   const Level& L = mg->lv[l];
   if (mg->use_bottom && mg->bottom_from >= 0 && static_cast<int>(l) >= mg->bottom_from)
     return bottom(mg, l, s);
   if (l + 1 == mg->lv.size()) return coarsest(mg, L, s);
   pm_status st;
+  if (use_legs(mg, l)) {
+    const Level& C = mg->lv[l + 1];
+    if ((st = leg_down(L, C, mg->d.pre_sweeps, s)) || (st = vcycle(mg, l + 1, s))) return st;
+    return leg_up(L, C, mg->d.post_sweeps, s);
+  }
   // small levels: one launch per sweep through L.tmp; an even number of sweeps in the cycle
   // leaves the result in L.phi
   const bool pp = mg->use_small_sweep && L.tmp && L.n <= kSmallSweepMax &&
@@ -2191,13 +2238,27 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
         return st;
       }
     }
-    if (L.n >= kSweepMin || (l > 0 && l + 1 < sizes.size() && L.n <= kSmallSweepMax)) {
+    if (L.n >= kSweepMin ||
+        (l > 0 && l + 1 < sizes.size() && L.n <= std::max(kSmallSweepMax, kLegMax))) {
       if ((st = dalloc(mg, reinterpret_cast<void**>(&L.tmp), bytes))) {
         destroy(mg);
         return st;
       }
     }
+    // faces below the finest level are zero for good; the legs write interior nodes only
+    for (float* q : {L.phi, L.rhs, L.tmp}) {
+      const hipError_t ze = l > 0 && q ? hipMemset(q, 0, bytes) : hipSuccess;
+      if (ze != hipSuccess) {
+        destroy(mg);
+        return pm::hip_fail("hipMemset (multigrid levels)", ze);
+      }
+    }
     mg->lv.push_back(L);
+  }
+  const hipError_t se = hipDeviceSynchronize();
+  if (se != hipSuccess) {
+    destroy(mg);
+    return pm::hip_fail("hipDeviceSynchronize (multigrid levels)", se);
   }
   // the bottom solver takes over at the first level <= kBottomMax when every level below it
   // is small too and the hierarchy fits its descriptor

@@ -375,3 +375,15 @@ def test_small_level_fused_sweep_equals_colour_passes(device, mode, n, sweeps, b
         out.append((phi.clone(), c0, s.last_cycles))
     assert torch.equal(out[0][0], out[1][0])
     assert out[0][1:] == out[1][1:]
+
+
+@pytest.mark.parametrize("mode,n,sweeps,bottom", [
+    ("mixed", 35, (2, 2), 1),    # 35 -> 18: blocks of one to eight interior nodes
+    ("mixed", 40, (1, 1), 0),    # even finest level, legs down to the 3^3 level
+    ("mixed", 74, (2, 1), 0),    # 74 -> 38 -> 19 -> 10 -> 5 -> 3: odd and even levels
+    ("mixed", 257, (2, 2), 1), ("mixed", 160, (1, 2), 1), ("mixed", 256, (1, 1), 1),
+    ("mixed", 142, (2, 2), 1)])  # 142 -> 72: the largest level with legs
+def test_one_launch_legs_equal_colour_passes(device, mode, n, sweeps, bottom):
+    """The V-cycle legs that run in one launch each (tile regions in LDS) give bitwise the phi
+    and the cycle counts of the per-pass kernels, cold and warm."""
+    test_small_level_fused_sweep_equals_colour_passes(device, mode, n, sweeps, bottom)
