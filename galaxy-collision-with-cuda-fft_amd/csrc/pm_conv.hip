@@ -233,10 +233,13 @@ struct ConvWgradArgs {
   int dz_c, kreal, nvox, chunks_per_split;
   float* partial;      // [splits][16*NR][kcols]
   int kcols;
+  float* partial_b;    // [splits][16*NR] channel sums of dz, or null
 };
 
 // grid (kcols/64, splits): one workgroup = 64 reduction columns x all output channels over
-// one voxel range; wave w owns columns 16w..16w+15.
+// one voxel range; wave w owns columns 16w..16w+15. The first column group's wave 0 also
+// multiplies dz with ones: the bias gradient's sums ride on operands it has loaded anyway
+// (a pass of their own took 31-118 us a layer at 64^3-16^3, as long as this kernel).
 template <int NR>
 __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
   constexpr int kLd = 40;  // 32 voxels + 8 pad (80-byte rows keep 16-byte alignment)
@@ -265,6 +268,11 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
   f32x4_t acc[NR];
 #pragma unroll
   for (int rb = 0; rb < NR; ++rb) acc[rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const bool sums = a.partial_b && blockIdx.x == 0 && wave == 0;
+  f32x4_t accb[NR];
+#pragma unroll
+  for (int rb = 0; rb < NR; ++rb) accb[rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const u32x4_t ones = u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
 
   const int vbeg = split * a.chunks_per_split * 32;
   const int vend = min(a.nvox, vbeg + a.chunks_per_split * 32);
@@ -301,7 +309,15 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
     for (int rb = 0; rb < NR; ++rb) {
       const u32x4_t aq = *reinterpret_cast<const u32x4_t*>(&sdz[16 * rb + row][8 * grp]);
       acc[rb] = mfma_bf16(aq, bq, acc[rb]);
+      if (sums) accb[rb] = mfma_bf16(aq, ones, accb[rb]);
     }
+  }
+  if (sums && row == 0) {  // every column holds the same sums
+#pragma unroll
+    for (int rb = 0; rb < NR; ++rb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a.partial_b[split * (16 * NR) + 16 * rb + 4 * grp + i] = accb[rb][i];
   }
   const int kcol = k0 + 16 * wave + row;
 #pragma unroll
@@ -313,53 +329,47 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
     }
 }
 
-// dw[co][ci][tap] (torch layout) = (accumulate ? dw : 0) + sum over splits in order.
-__global__ void __launch_bounds__(256) wgrad_fold_kernel(const float* __restrict__ partial,
-                                                         int splits, int cout, int rows,
-                                                         int kcols, int cin, float* dw,
-                                                         int accumulate) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int total = cout * cin * 27;
-  if (idx >= total) return;
-  const int co = idx / (cin * 27);
-  const int rem = idx - co * cin * 27;
-  const int c = rem / 27, tap = rem - c * 27;
-  const int k = tap * cin + c;
-  float s = 0.0f;
-  for (int sp = 0; sp < splits; ++sp) s += partial[(static_cast<int64_t>(sp) * rows + co) * kcols + k];
-  dw[idx] = accumulate ? dw[idx] + s : s;
-}
-
-// Per-block channel sums of dz[v][c] (c < cout) over a voxel range -> partial[block][c].
-__global__ void __launch_bounds__(256) channel_sum_kernel(const uint16_t* __restrict__ dz,
-                                                          int nvox, int dz_c, int cout,
-                                                          int vox_per_block,
-                                                          float* __restrict__ partial) {
-  __shared__ float red[256];
-  const int tid = threadIdx.x;
-  const int lanes = 256 / dz_c;  // dz_c is a power of two in [8, 128]
-  const int c = tid % dz_c, l = tid / dz_c;
-  const int v0 = blockIdx.x * vox_per_block;
-  const int v1 = min(nvox, v0 + vox_per_block);
-  float s = 0.0f;
-  for (int v = v0 + l; v < v1; v += lanes) s += bf2f(dz[static_cast<int64_t>(v) * dz_c + c]);
-  red[tid] = s;
-  __syncthreads();
-  if (l == 0 && c < cout) {
-    float t = 0.0f;
-    for (int j = 0; j < lanes; ++j) t += red[j * dz_c + c];
-    partial[static_cast<int64_t>(blockIdx.x) * cout + c] = t;
+// dw[co][ci][tap] (torch layout) = (accumulate ? dw : 0) + the sum over splits, and db[co] the
+// same of the channel sums. grid (kcols/64, cout + 1): 64 columns of one output channel (the
+// last grid row: 64 channels of the bias); the kFoldWaves waves take every kFoldWaves-th split,
+// a few loads in flight at once, and their sums are added in wave order (deterministic). One
+// thread that walked all splits of an output kept a load at a time in flight: 80 us for the
+// 283 splits of a 64^3 layer of 16 channels, 157 us for 512.
+constexpr int kFoldWaves = 16;
+__global__ void __launch_bounds__(64 * kFoldWaves) wgrad_fold_kernel(
+    const float* __restrict__ partial, const float* __restrict__ partial_b, int splits, int cout,
+    int rows, int kcols, int cin, float* dw, float* db, int accumulate) {
+  __shared__ float s[kFoldWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = static_cast<int>(blockIdx.x) * 64 + lane;
+  const bool bias = static_cast<int>(blockIdx.y) == cout;
+  const int co = bias ? col : static_cast<int>(blockIdx.y);
+  const bool live = bias ? db && col < cout : col < 27 * cin;
+  const float* src = bias ? partial_b + col : partial + static_cast<int64_t>(co) * kcols + col;
+  const int64_t stride = bias ? rows : static_cast<int64_t>(rows) * kcols;
+  float sum = 0.0f;
+  if (live) {
+    constexpr int kAhead = 8;
+    for (int sp = wave; sp < splits; sp += kFoldWaves * kAhead) {
+      float v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int at = sp + u * kFoldWaves;
+        v[u] = at < splits ? src[at * stride] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) sum += v[u];
+    }
   }
-}
-
-__global__ void __launch_bounds__(256) channel_fold_kernel(const float* __restrict__ partial,
-                                                           int blocks, int cout, float* db,
-                                                           int accumulate) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cout) return;
-  float s = 0.0f;
-  for (int b = 0; b < blocks; ++b) s += partial[static_cast<int64_t>(b) * cout + c];
-  db[c] = accumulate ? db[c] + s : s;
+  s[wave][lane] = sum;
+  __syncthreads();
+  if (wave != 0 || !live) return;
+  float t = s[0][lane];
+#pragma unroll
+  for (int w = 1; w < kFoldWaves; ++w) t += s[w][lane];
+  float* out = bias ? db + col
+                    : dw + (static_cast<int64_t>(co) * cin + col % cin) * 27 + col / cin;
+  *out = accumulate ? *out + t : t;
 }
 
 // Pack torch-layout float32 weights w[co][ci][27] into bf16 GEMM operands.
@@ -586,8 +596,7 @@ int64_t wgrad_partial_floats(int cin, int cout, int r) {
   wgrad_plan(cin, cout, r, &splits, &chunks);
   const int kcols = (kpad(cin) + 63) / 64 * 64;
   const int rows = rows_pad(store_channels(cout));
-  const int64_t bias_floats = (static_cast<int64_t>(r) * r * r + 2047) / 2048 * cout;
-  return std::max(static_cast<int64_t>(splits) * rows * kcols, bias_floats);
+  return static_cast<int64_t>(splits) * rows * (kcols + 1);  // and the channel sums
 }
 
 void wgrad_plan(int cin, int cout, int r, int* splits, int* chunks_per_split) {
@@ -635,6 +644,8 @@ pm_status wgrad(const uint16_t* xa, int ca, const uint16_t* xb, int cb, int r, i
   a.partial = partial;
   a.kcols = (kpad(cin) + 63) / 64 * 64;
   const int nr = std::max(1, rows_pad(dz_c) / 16);  // 1, 2, 4 or 8 (dz_c is 8..128)
+  const int rows = 16 * nr;
+  a.partial_b = db ? partial + static_cast<int64_t>(splits) * rows * a.kcols : nullptr;
   const dim3 grid(static_cast<unsigned>(a.kcols / 64), static_cast<unsigned>(splits));
   {
     const double flops = 2.0 * 27.0 * cin * cout * static_cast<double>(a.nvox);
@@ -647,24 +658,10 @@ pm_status wgrad(const uint16_t* xa, int ca, const uint16_t* xb, int cb, int r, i
     }
     PM_CHECK_LAUNCH("conv_wgrad_kernel");
   }
-  const int rows = 16 * nr;
-  const int total = cout * cin * 27;
-  wgrad_fold_kernel<<<pm::blocks_for(total), 256, 0, s>>>(partial, splits, cout, rows, a.kcols,
-                                                           cin, dw, accumulate);
+  const dim3 fold(static_cast<unsigned>(a.kcols / 64), static_cast<unsigned>(cout + (db ? 1 : 0)));
+  wgrad_fold_kernel<<<fold, 64 * kFoldWaves, 0, s>>>(partial, a.partial_b, splits, cout, rows,
+                                                     a.kcols, cin, dw, db, accumulate);
   PM_CHECK_LAUNCH("wgrad_fold_kernel");
-  if (db) {
-    // bias gradient: channel sums of dz, reusing the front of the partial buffer
-    const int64_t nvox = a.nvox;
-    const int vpb = 2048;
-    const int blocks = static_cast<int>((nvox + vpb - 1) / vpb);
-    PM_REQUIRE(static_cast<int64_t>(blocks) * cout <= partial_floats,
-               "pm_conv3d_bwd_weight_bf16: partial buffer too small for the bias gradient");
-    // the weight fold above reads `partial` on the same stream first, so reuse is ordered
-    channel_sum_kernel<<<blocks, 256, 0, s>>>(dz, a.nvox, dz_c, cout, vpb, partial);
-    PM_CHECK_LAUNCH("channel_sum_kernel");
-    channel_fold_kernel<<<pm::blocks_for(cout), 256, 0, s>>>(partial, blocks, cout, db, accumulate);
-    PM_CHECK_LAUNCH("channel_fold_kernel");
-  }
   return PM_OK;
 }
 
