@@ -49,7 +49,7 @@ struct ConvFwdArgs {
   const uint16_t* xa;
   const uint16_t* xb;
   int ca, cb, cin, r, ra, up;
-  const uint16_t* w;  // packed [rows][kpad]
+  const uint16_t* w;  // packed operands (pack_weights_kernel)
   int kpad, kreal, rows;
   int kc_per;         // 32-wide reduction chunks per split (blockIdx.z)
   float* partial;     // split-K: raw sums [split][r^3][rows] (epilogue in a second kernel)
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvFwdArgs a) {
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     wvalid[nb] = co0 + 16 * nb < a.rows;
-    wrow[nb] = a.w + static_cast<int64_t>(wvalid[nb] ? co0 + 16 * nb + row : 0) * a.kpad + 8 * grp;
+    wrow[nb] = a.w + static_cast<int64_t>(wvalid[nb] ? co0 + 16 * nb : 0) * a.kpad + 8 * lane;
   }
 
   // G consecutive 32-wide chunks per round: every operand load of the round is issued
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvFwdArgs a) {
       }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
-        bv[g][nb] = (live && wvalid[nb]) ? load16(wrow[nb] + kcg) : u32x4_t{0u, 0u, 0u, 0u};
+        bv[g][nb] = (live && wvalid[nb]) ? load16(wrow[nb] + 16 * kcg) : u32x4_t{0u, 0u, 0u, 0u};
       ci += 32;
       while (ci >= a.cin) {
         ci -= a.cin;
@@ -191,6 +191,182 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvFwdArgs a) {
       for (int i = 0; i < 4; ++i) {
         const int v = vbase + 16 * mb + 4 * grp + i;
         if (v >= nvox) continue;
+        float val = 0.0f;
+        if (real) {
+          val = acc[mb][nb][i] + b;
+          if (a.act && !(val > 0.0f)) val = val * a.slope;
+        }
+        if (a.y) a.y[static_cast<int64_t>(v) * a.cout_st + co] = f2bf(val);
+        if (a.y32 && real) a.y32[static_cast<int64_t>(v) * a.cout + co] = val;
+      }
+    }
+  }
+}
+
+// The forward convolution from an LDS tile: a workgroup stages the input of a 2 x 8 x 8 block of
+// output voxels with its halo once (4 x 10 x 10 voxels, all CIN input channels) and its waves
+// read every tap's operand from there, where conv_fwd_kernel loads each activation 27 times
+// through the caches and decodes its address each time (us, both with 256 threads: 16 -> 16 at
+// 64^3 24 there, 12 here; 48 -> 16 at 64^3 54, 27; 96 -> 32 at 32^3 37 + 5 for its split sums, 17;
+// 128 -> 128 at 8^3 10 + 9, 19; 192 -> 64 at 16^3 25 + 5, 28). Bound: LDS operand reads and the
+// staging's latency. Wave w computes voxels 32 w .. 32 w + 31
+// x 16 * NB output channels over the reduction in packed order, as one split of conv_fwd_kernel
+// does. The reduction is unrolled: a chunk of 32 is one weight load, two LDS reads and 2 * NB
+// MFMAs, its addresses constant offsets (computed per chunk, in vector or scalar registers, they
+// took several times as long as the MFMAs). A voxel's channels are padded by 16 bytes so that
+// the 16 rows of an operand read fall into different banks.
+constexpr int kHaloY = 10, kHaloZ = 100;   // strides of the staged 4 x 10 x 10 voxels
+constexpr int kHaloVox = 400;
+
+constexpr int tap_offset(int tap) {  // staged voxels from the block's first; taps past 26 read one
+  return tap > 26 ? 0 : (tap / 9) * kHaloZ + (tap / 3 % 3) * kHaloY + tap % 3;
+}
+
+struct ConvTileArgs {
+  ConvFwdArgs c;
+  pm::FastDiv dt;         // 8 x 8 blocks of a plane per axis
+};
+
+// S > 1: the channels are staged in S slices, one after the other (less LDS, so that another
+// workgroup computes while this one stages).
+template <int CIN, int NB, int S>
+__global__ void __launch_bounds__(256) conv_tile_kernel(ConvTileArgs t) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  constexpr int CS = CIN / S;  // channels staged at once
+  static_assert(S == 1 || CS % 32 == 0, "a slice is whole chunks of every tap");
+  constexpr int kPitch = 2 * CS + 16;
+  constexpr int kReal = 27 * CS, kChunks = (kReal + 31) / 32;  // of a slice
+  const ConvFwdArgs& a = t.c;
+  const int r = a.r;
+  const uint32_t blk = static_cast<uint32_t>(pm::xcd_block());
+  const uint32_t q0 = pm::fast_div(blk, t.dt), q1 = pm::fast_div(q0, t.dt);
+  const int x0 = static_cast<int>(blk - q0 * t.dt.d) * 8;
+  const int y0 = static_cast<int>(q0 - q1 * t.dt.d) * 8;
+  const int z0 = static_cast<int>(q1) * 2;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane & 15, grp = lane >> 4;
+  const int co0 = static_cast<int>(blockIdx.y) * 16 * NB;
+  // weights of the first chunks leave before the staging
+  constexpr int kAhead = NB == 1 ? 8 : 4;
+  const uint16_t* wrow[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)  // a column block past the packed rows repeats the last one
+    wrow[nb] = a.w + static_cast<int64_t>(min(co0 + 16 * nb, a.rows - 16)) * a.kpad + 8 * lane;
+  u32x4_t bv[kAhead][NB];
+  // weights of chunk c of slice s: all of a tap's channels are consecutive chunks
+  auto weights = [&](int s, int c, u32x4_t (&dst)[NB]) {
+    const int at = S == 1 ? c : c / (CS / 32) * (CIN / 32) + s * (CS / 32) + c % (CS / 32);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) dst[nb] = load16(wrow[nb] + 512 * at);
+  };
+  const unsigned char* base[2];
+  const bool second = grp >= 2;
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int m = 32 * wave + 16 * mb + row;
+    base[mb] = lds + ((m >> 6) * kHaloZ + ((m >> 3) & 7) * kHaloY + (m & 7)) * kPitch;
+  }
+  f32x4_t acc[2][NB];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int slice = 0; slice < S; ++slice) {
+#pragma unroll
+    for (int c = 0; c < kAhead && c < kChunks; ++c) weights(slice, c, bv[c]);
+    if (slice > 0) __syncthreads();  // the previous slice has been read
+    {
+      // thread -> one (x, 8 channels) of a staged row and every kRows-th of the 40 rows: source
+      // tensor, channel and x are found once
+      constexpr int kItems = kHaloY * (CS / 8), kRows = 256 / kItems;
+      constexpr int kRounds = (40 + kRows - 1) / kRows;
+      constexpr int kBatch = kRounds < 10 ? kRounds : 10;  // loads in flight per thread
+      const int rr = static_cast<int>(threadIdx.x) / kItems;
+      const int item = static_cast<int>(threadIdx.x) - rr * kItems;
+      const int hx = item / (CS / 8), c8 = 8 * (item - hx * (CS / 8)), g8 = slice * CS + c8;
+      const bool from_a = g8 < a.ca;
+      const int sh = from_a ? a.up : 0, rs = from_a ? a.ra : r, cs = from_a ? a.ca : a.cb;
+      const int x = x0 + hx - 1;
+      const uint16_t* src = (from_a ? a.xa + g8 : a.xb + (g8 - a.ca)) + (x >> sh) * cs;
+      const bool x_in = rr < kRows && x >= 0 && x < r;
+      unsigned char* dst = lds + hx * kPitch + 2 * c8;
+#pragma unroll
+      for (int u0 = 0; u0 < kRounds; u0 += kBatch) {
+        u32x4_t v[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          const int rowi = rr + (u0 + u) * kRows;
+          const int hz = (rowi * 205) >> 11, hy = rowi - 10 * hz;  // rowi / 10 for rowi < 80
+          const int z = z0 + hz - 1, y = y0 + hy - 1;
+          const bool in = u0 + u < kRounds && rowi < 40 && x_in && z >= 0 && z < r && y >= 0 && y < r;
+          const int vrow = __mul24(__mul24(z >> sh, rs) + (y >> sh), rs);
+          v[u] = in ? load16(src + static_cast<int64_t>(vrow) * cs) : u32x4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          const int rowi = rr + (u0 + u) * kRows;
+          if (u0 + u < kRounds && rowi < 40 && rr < kRows)
+            *reinterpret_cast<u32x4_t*>(dst + rowi * (kHaloY * kPitch)) = v[u];
+        }
+      }
+    }
+    __syncthreads();
+    // operand address of row block mb: base + the chunk's constant; where the chunk's two halves
+    // (16 channels each) lie in different taps, the lanes of the second half add the taps'
+    // distance: one voxel along x, or to the next row or plane
+    constexpr int kReads = 3;  // chunks whose LDS reads are under way
+    u32x4_t av[kReads][2];
+    auto operand = [&](int c, u32x4_t (&dst)[2]) {
+      // byte offsets of the chunk's four operand groups (8 channels each)
+      int off[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int k = 32 * c + 8 * g;
+        off[g] = tap_offset(k / CS) * kPitch + 2 * (k % CS);
+      }
+      int lane_off;
+      if (CS % 16 == 0) {
+        const int jump = off[2] - off[0] - 32;  // 0 where the chunk lies in one tap
+        lane_off = 16 * grp + (second ? jump : 0) + off[0];
+      } else {
+        lane_off = grp == 0 ? off[0] : grp == 1 ? off[1] : grp == 2 ? off[2] : off[3];
+      }
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) dst[mb] = *reinterpret_cast<const u32x4_t*>(base[mb] + lane_off);
+      if (32 * (c + 1) > kReal) {  // the last chunk's padding: weights there are zero, so must x be
+        const bool in = 32 * c + 8 * grp < kReal;
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) dst[mb] = in ? dst[mb] : u32x4_t{0u, 0u, 0u, 0u};
+      }
+    };
+#pragma unroll
+    for (int c = 0; c < kReads && c < kChunks; ++c) operand(c, av[c]);
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          acc[mb][nb] = mfma_bf16(av[c % kReads][mb], bv[c % kAhead][nb], acc[mb][nb]);
+      if (c + kReads < kChunks) operand(c + kReads, av[c % kReads]);
+      if (c + kAhead < kChunks) weights(slice, c + kAhead, bv[c % kAhead]);
+    }
+  }
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    const int co = co0 + 16 * nb + row;
+    if (co >= a.cout_st) continue;
+    const bool real = co < a.cout;
+    const float b = (real && a.bias) ? a.bias[co] : 0.0f;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = 32 * wave + 16 * mb + 4 * grp + i;
+        const int z = z0 + (m >> 6), y = y0 + ((m >> 3) & 7), x = x0 + (m & 7);
+        if (z >= r || y >= r || x >= r) continue;
+        const int v = (z * r + y) * r + x;
         float val = 0.0f;
         if (real) {
           val = acc[mb][nb][i] + b;
@@ -375,14 +551,19 @@ __global__ void __launch_bounds__(64 * kFoldWaves) wgrad_fold_kernel(
 // Pack torch-layout float32 weights w[co][ci][27] into bf16 GEMM operands.
 //   forward:   wp[co][tap*cin + ci]            rows co < rows_pad, k < kpad
 //   transpose: wp[ci][tap'*cout_st + co] = w[co][ci][26 - tap']   (backward-data operand)
+// stored by MFMA operand: 16 rows x 32 k are 512 consecutive values, lane 16 * (k / 8 % 4) +
+// row % 16 holding 8 of them, so that a wave loads an operand as one contiguous kilobyte (as
+// 16 rows of 64 bytes it kept the cache port busy for longer than the MFMAs took).
 __global__ void __launch_bounds__(256) pack_weights_kernel(const float* __restrict__ w, int cout,
                                                            int cin, int transpose, int cin_eff,
                                                            int rows_pad, int kpad,
                                                            uint16_t* __restrict__ wp) {
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (idx >= static_cast<int64_t>(rows_pad) * kpad) return;
-  const int rrow = static_cast<int>(idx / kpad);
-  const int k = static_cast<int>(idx - static_cast<int64_t>(rrow) * kpad);
+  const int lane = static_cast<int>(idx >> 3) & 63, chunks = kpad >> 5;
+  const int block = static_cast<int>(idx >> 9);
+  const int rrow = block / chunks * 16 + (lane & 15);
+  const int k = block % chunks * 32 + (lane >> 4) * 8 + static_cast<int>(idx & 7);
   float v = 0.0f;
   if (k < 27 * cin_eff) {
     const int tap = k / cin_eff, c = k - tap * cin_eff;
@@ -530,6 +711,51 @@ FwdPlan fwd_plan(int nvox, int rows, int kpad_, bool allow_split) {
   return p;
 }
 
+// Input channel counts that conv_tile_kernel is built for (192 fill the LDS).
+bool tile_fits(int cin) {
+  switch (cin) {
+    case 8: case 16: case 32: case 48: case 64: case 96: case 128: case 192: return true;
+    default: return false;
+  }
+}
+
+template <int CIN, int S>
+void launch_tile(const ConvTileArgs& t, int nb, dim3 grid, hipStream_t s) {
+  constexpr size_t lds = static_cast<size_t>(kHaloVox) * (2 * CIN / S + 16);
+  static_assert(lds <= 160 * 1024, "the tile fits the LDS");
+  if (nb == 1) conv_tile_kernel<CIN, 1, S><<<grid, 256, lds, s>>>(t);
+  else if (nb == 2) conv_tile_kernel<CIN, 2, S><<<grid, 256, lds, s>>>(t);
+  else conv_tile_kernel<CIN, 3, S><<<grid, 256, lds, s>>>(t);
+}
+
+pm_status fwd_tile(const ConvFwdArgs& a, const char* timer, hipStream_t s) {
+  const int tx = (a.r + 7) / 8, tz = (a.r + 1) / 2;
+  ConvTileArgs t;
+  t.c = a;
+  t.c.partial = nullptr;
+  t.dt = pm::make_fast_div(static_cast<uint32_t>(tx));
+  const int blocks = a.rows / 16;
+  const int64_t tiles = static_cast<int64_t>(tx) * tx * tz;
+  // column blocks per workgroup: as many as leave two workgroups per CU
+  int nb = std::min(3, blocks);
+  while (nb > 1 && tiles * ((blocks + nb - 1) / nb) < 512) --nb;
+  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>((blocks + nb - 1) / nb));
+  const double flops = 2.0 * 27.0 * a.cin * a.cout * static_cast<double>(a.r) * a.r * a.r;
+  PM_TIMED(timer, flops, s);
+  switch (a.cin) {
+    case 8: launch_tile<8, 1>(t, nb, grid, s); break;
+    case 16: launch_tile<16, 1>(t, nb, grid, s); break;
+    case 32: launch_tile<32, 1>(t, nb, grid, s); break;
+    case 48: launch_tile<48, 1>(t, nb, grid, s); break;
+    case 64: launch_tile<64, 1>(t, nb, grid, s); break;
+    case 96: launch_tile<96, 3>(t, nb, grid, s); break;
+    case 128: launch_tile<128, 1>(t, nb, grid, s); break;
+    default: launch_tile<192, 2>(t, nb, grid, s); break;
+  }
+  PM_CHECK_LAUNCH("conv_tile_kernel");
+  return PM_OK;
+}
+
 int64_t fwd_scratch_floats(int cin, int cout, int r) {
   const int64_t nvox = static_cast<int64_t>(r) * r * r;
   const FwdPlan p = fwd_plan(static_cast<int>(nvox), rows_pad(cout), kpad(cin), true);
@@ -566,6 +792,7 @@ pm_status fwd(const uint16_t* xa, int ca, const uint16_t* xb, int cb, int r, int
   a.y = y;
   a.y32 = y32;
   const int nvox = r * r * r;
+  if (tile_fits(a.cin)) return fwd_tile(a, timer, s);
   FwdPlan p = fwd_plan(nvox, a.rows, a.kpad, scratch != nullptr);
   if (p.ksplit > 1 && static_cast<int64_t>(p.ksplit) * nvox * a.rows > scratch_floats)
     p = fwd_plan(nvox, a.rows, a.kpad, false);

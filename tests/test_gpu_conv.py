@@ -259,3 +259,20 @@ def test_conv_argument_checks(device):
         nat.call("pm_conv3d_fwd_bf16", nat.ptr(x, torch.bfloat16), 12, None, 0, 8, 0,
                  nat.ptr(x, torch.bfloat16), None, 16, 0, 0.0, nat.ptr(x, torch.bfloat16), None,
                  None, 0, nat.stream())
+
+
+@pytest.mark.parametrize("r,ca,cb,up,cout,act", [
+    (9, 8, 0, 0, 24, 1),       # one voxel past a tile on every axis; 8 channels: lane offsets
+    (10, 16, 0, 0, 48, 0),     # three column blocks in one workgroup
+    (1, 32, 0, 0, 16, 1),      # a tile that is nearly all padding
+    (3, 48, 0, 0, 16, 1),      # chunks whose halves lie in different taps
+    (12, 64, 32, 1, 32, 1),    # 96 staged in three slices, upsampled ++ skip across slices
+    (7, 96, 96, 0, 64, 1),     # 192 in two slices, slice border between the tensors
+    (5, 128, 0, 0, 192, 0),
+    (17, 64, 0, 0, 8, 1),
+    (6, 24, 0, 0, 16, 1),      # channel counts without a tile kernel
+    (4, 128, 128, 0, 16, 0),
+])
+def test_conv_tile_edges_match_float64(device, r, ca, cb, up, cout, act):
+    """Tile borders, halves of a chunk in two taps, channel slices and the fallback."""
+    test_conv_forward_matches_float64(device, r, ca, cb, up, cout, act, False)
