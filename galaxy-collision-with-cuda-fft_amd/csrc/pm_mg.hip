@@ -1031,7 +1031,8 @@ __device__ __forceinline__ void quad_nbr_sums(const float* __restrict__ eo, uint
   quad_nbr_sum(quad_nbr_load(eo, t0, nh, hn, p), p, s);
 }
 
-template <bool ZERO>
+// FACES: the array's faces hold values (PLAIN's phi) and keep them; otherwise they are zero.
+template <bool ZERO, bool FACES = false>
 __global__ void __launch_bounds__(256) rbs4_kernel(float* __restrict__ e,
                                                    const float* __restrict__ r, int n, int hn,
                                                    float h2, int color) {
@@ -1050,14 +1051,17 @@ __global__ void __launch_bounds__(256) rbs4_kernel(float* __restrict__ e,
     nb = quad_nbr_load(e + (plane - own), q.t0, static_cast<uint32_t>(n) * hn,
                        static_cast<uint32_t>(hn), p);
   const float4 rr = ld4(r, own + q.t0);
+  // a row's two end nodes are faces: one of them lies in this quad's first or last position
+  const bool end = FACES && (q.kk0 == 0 || q.kk0 + 4 == hn);
+  const float4 old = end ? ld4(e, own + q.t0) : make_float4(0.f, 0.f, 0.f, 0.f);
   __builtin_amdgcn_sched_barrier(0);  // all loads leave before any arithmetic
   if (!ZERO) quad_nbr_sum(nb, p, s);
   float out[4];
 #pragma unroll
   for (int k4 = 0; k4 < 4; ++k4) {
     const int k = 2 * (q.kk0 + k4) + p;
-    // faces (k = 0, k = n-1) and pad slots keep their zero
-    out[k4] = (k >= 1 && k <= n - 2) ? (s[k4] - h2 * at4(rr, k4)) / 6.0f : 0.0f;
+    // faces (k = 0, k = n-1) and pad slots keep their value
+    out[k4] = (k >= 1 && k <= n - 2) ? (s[k4] - h2 * at4(rr, k4)) / 6.0f : at4(old, k4);
   }
   *reinterpret_cast<float4*>(e + own + q.t0) = make_float4(out[0], out[1], out[2], out[3]);
 }
@@ -1234,6 +1238,9 @@ __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* 
     const Quad& qq = q[m];
     const int p = (qq.i + qq.j + 1) & 1;  // parity of k; k>>1 = kk0 + e
     const int ci = qq.i >> 1, cj = qq.j >> 1, oi = qq.i & 1, oj = qq.j & 1;
+    // the fifth coarse value serves odd k; on a halving level the last quad's lies past the row
+    // (only the face k = n - 1 would take it)
+    const bool fifth = p && qq.kk0 + 4 < nc;
     float c[2][2][5];
 #pragma unroll
     for (int di = 0; di < 2; ++di) {
@@ -1244,12 +1251,12 @@ __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* 
           const int row = ((ci + di - ci0) * ncj + (cj + dj - cj0)) * nc + qq.kk0;
 #pragma unroll
           for (int x = 0; x < 5; ++x)
-            c[di][dj][x] = (need && (x < 4 || p)) ? s_c[row + x] : 0.0f;
+            c[di][dj][x] = (need && (x < 4 || fifth)) ? s_c[row + x] : 0.0f;
         } else {
           const uint32_t row = (ci + di) * nc2 + static_cast<uint32_t>(cj + dj) * nc + qq.kk0;
 #pragma unroll
           for (int x = 0; x < 5; ++x)
-            c[di][dj][x] = (need && (x < 4 || p)) ? phi_c[row + x] : 0.0f;
+            c[di][dj][x] = (need && (x < 4 || fifth)) ? phi_c[row + x] : 0.0f;
         }
       }
     }
@@ -1456,6 +1463,84 @@ __global__ void __launch_bounds__(256) to_split_kernel(const float* __restrict__
   const pm::Idx3 q3 = pm::idx3(c, n);
   dst[static_cast<int64_t>((q3.i + q3.j + q3.k) & 1) * n2 * hn +
       (static_cast<int64_t>(q3.i) * n + q3.j) * hn + (q3.k >> 1)] = src[c];
+}
+
+// natural <-> split copies of 8 consecutive nodes per thread (n % 8 == 0, 16-byte aligned).
+__global__ void __launch_bounds__(256) to_split4_kernel(const float* __restrict__ src,
+                                                        float* __restrict__ dst, int n, int hn) {
+  const int hq = hn >> 2;
+  const uint32_t quads = static_cast<uint32_t>(n) * n * hq;
+  const int64_t u = pm::xcd_block() * blockDim.x + threadIdx.x;
+  if (u >= quads) return;
+  const Quad q = quad_idx(static_cast<uint32_t>(u), n, hq);
+  const uint32_t c = static_cast<uint32_t>(u) * 8u, plane = static_cast<uint32_t>(n) * n * hn;
+  const float4 a = ld4(src, c), b = ld4(src, c + 4);
+  const float4 even = make_float4(a.x, a.z, b.x, b.z), odd = make_float4(a.y, a.w, b.y, b.w);
+  const bool p = ((q.i + q.j) & 1) != 0;  // the even nodes have colour p
+  *reinterpret_cast<float4*>(dst + q.t0) = p ? odd : even;
+  *reinterpret_cast<float4*>(dst + plane + q.t0) = p ? even : odd;
+}
+
+__global__ void __launch_bounds__(256) from_split4_kernel(const float* __restrict__ src,
+                                                          float* __restrict__ dst, int n,
+                                                          int hn) {
+  const int hq = hn >> 2;
+  const uint32_t quads = static_cast<uint32_t>(n) * n * hq;
+  const int64_t u = pm::xcd_block() * blockDim.x + threadIdx.x;
+  if (u >= quads) return;
+  const Quad q = quad_idx(static_cast<uint32_t>(u), n, hq);
+  const uint32_t c = static_cast<uint32_t>(u) * 8u, plane = static_cast<uint32_t>(n) * n * hn;
+  const float4 v0 = ld4(src, q.t0), v1 = ld4(src, plane + q.t0);
+  const bool p = ((q.i + q.j) & 1) != 0;
+  const float4 even = p ? v1 : v0, odd = p ? v0 : v1;
+  *reinterpret_cast<float4*>(dst + c) = make_float4(even.x, odd.x, even.y, odd.y);
+  *reinterpret_cast<float4*>(dst + c + 4) = make_float4(even.z, odd.z, even.w, odd.w);
+}
+
+// residual_sumsq_kernel from the split layout: the same float32 residuals, summed in another
+// order (float64).
+__global__ void __launch_bounds__(256) residual_sumsq_s4_kernel(const float* __restrict__ e,
+                                                                const float* __restrict__ r, int n,
+                                                                int hn, float inv_h2,
+                                                                double* __restrict__ partials) {
+  __shared__ double s_red[4];
+  double v[1] = {0.0};
+  const int hq = hn >> 2;
+  const int64_t quads = static_cast<int64_t>(n) * n * hq;
+  const uint32_t plane = static_cast<uint32_t>(n) * n * hn, nh = static_cast<uint32_t>(n) * hn;
+  int64_t r_begin, r_end;
+  pm::block_range(quads, r_begin, r_end);
+  for (int64_t u = r_begin + threadIdx.x; u < r_end; u += blockDim.x) {
+    const Quad q = quad_idx(static_cast<uint32_t>(u), n, hq);
+    if (q.i < 1 || q.i > n - 2 || q.j < 1 || q.j > n - 2) continue;
+    NbrQuad nb[2];
+    float4 ev[2], rv[2];
+#pragma unroll
+    for (int color = 0; color < 2; ++color) {
+      const uint32_t own = static_cast<uint32_t>(color) * plane;
+      nb[color] = quad_nbr_load(e + (plane - own), q.t0, nh, static_cast<uint32_t>(hn),
+                                (q.i + q.j + color) & 1);
+      ev[color] = ld4(e, own + q.t0);
+      rv[color] = ld4(r, own + q.t0);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all loads leave before any arithmetic
+#pragma unroll
+    for (int color = 0; color < 2; ++color) {
+      const int p = (q.i + q.j + color) & 1;
+      float s[4];
+      quad_nbr_sum(nb[color], p, s);
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4) {
+        const int k = 2 * (q.kk0 + k4) + p;
+        const float lap = (s[k4] - 6.0f * at4(ev[color], k4)) * inv_h2;
+        const double x = static_cast<double>(at4(rv[color], k4) - lap);
+        const double acc = v[0] + x * x;
+        v[0] = (k >= 1 && k <= n - 2) ? acc : v[0];
+      }
+    }
+  }
+  pm::block_sum<1>(v, s_red);
+  if (threadIdx.x == 0) partials[blockIdx.x * pm::kRedMaxQ] = v[0];
 }
 
 struct Level {
@@ -1905,6 +1990,47 @@ pm_status vcycle_split0(pm_mg* mg, float* phi, int carry, hipStream_t s) {
   return PM_OK;
 }
 
+// PLAIN's cycle with the finest level in split layout: e0s holds phi (faces included), r32s the
+// right-hand side; post_sweeps >= 1, so the colour-0 nodes need no prolongation (their next
+// pass does not read them).
+pm_status vcycle_plain_split(pm_mg* mg, hipStream_t s) {
+  const Level& L = mg->lv[0];
+  const Level& C = mg->lv[1];
+  const int n = L.n, hn = mg->hn;
+  const int64_t quads = static_cast<int64_t>(n) * n * hn / 4;
+  const double nodes = static_cast<double>(L.nodes());
+  float* e = mg->e0s;
+  const float* r = mg->r32s;
+  auto sweeps = [&](int count) -> pm_status {
+    for (int q = 0; q < 2 * count; ++q) {
+      PM_TIMED(level_name("mg.rbs", n), 6.0 * nodes, s);
+      rbs4_kernel<false, true><<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, q & 1);
+      PM_CHECK_LAUNCH("rbs4_kernel");
+    }
+    return PM_OK;
+  };
+  pm_status st;
+  if ((st = sweeps(mg->d.pre_sweeps))) return st;
+  {
+    PM_TIMED(level_name("mg.residual_s", n), kResidualBytes * nodes, s);
+    residual_s4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, L.res, n, hn, L.inv_h2);
+    PM_CHECK_LAUNCH("residual_s4_kernel");
+  }
+  {
+    PM_TIMED(level_name("mg.restrict", n), kRestrictBytes * nodes, s);
+    restrict_kernel<<<pm::blocks_for(C.nodes()), pm::kBlock, 0, s>>>(L.res, C.rhs, C.phi, n, C.n);
+    PM_CHECK_LAUNCH("restrict_kernel");
+  }
+  if ((st = vcycle(mg, 1, s))) return st;
+  {
+    PM_TIMED(level_name("mg.prolong_s", n), 4.0 * nodes, s);
+    prolong_s4_kernel<<<pm::blocks_for((quads + kProlongQ - 1) / kProlongQ), pm::kBlock, 0, s>>>(
+        C.phi, e, n, hn, C.n);
+    PM_CHECK_LAUNCH("prolong_s4_kernel");
+  }
+  return sweeps(mg->d.post_sweeps);
+}
+
 // Copies `count` float64 results from the device (synchronizes the stream).
 pm_status read_scalars(pm_mg* mg, const double* dev, int count, double* out, hipStream_t s) {
   PM_TRY_HIP(hipMemcpyAsync(mg->host, dev, sizeof(double) * count, hipMemcpyDeviceToHost, s));
@@ -1914,12 +2040,18 @@ pm_status read_scalars(pm_mg* mg, const double* dev, int count, double* out, hip
 }
 
 // ||rhs - A phi|| over the finest level (float32 residual, float64 sum), synchronizing.
-pm_status plain_residual_norm(pm_mg* mg, const float* phi, double* out, hipStream_t s) {
+// split: phi and the right-hand side lie in e0s and r32s.
+pm_status plain_residual_norm(pm_mg* mg, const float* phi, double* out, hipStream_t s,
+                              bool split = false) {
   const Level& L = mg->lv[0];
   const unsigned b = pm::red_blocks(L.nodes());
   {
     PM_TIMED("mg.residual_norm", 8.0 * L.nodes(), s);
-    residual_sumsq_kernel<<<b, pm::kBlock, 0, s>>>(phi, mg->f0, L.n, L.inv_h2, mg->partials);
+    if (split)
+      residual_sumsq_s4_kernel<<<b, pm::kBlock, 0, s>>>(mg->e0s, mg->r32s, L.n, mg->hn, L.inv_h2,
+                                                        mg->partials);
+    else
+      residual_sumsq_kernel<<<b, pm::kBlock, 0, s>>>(phi, mg->f0, L.n, L.inv_h2, mg->partials);
     PM_CHECK_LAUNCH("residual_sumsq_kernel");
   }
   pm::fold_partials_kernel<1><<<1, pm::kBlock, 0, s>>>(mg->partials, static_cast<int>(b),
@@ -1982,7 +2114,8 @@ enum {
   kCycleCarryFirst = 2,
   kCycleCarryMore = 3,
   kCycleCarryFirstFold = 4,
-  kCycleCarryMoreFold = 5
+  kCycleCarryMoreFold = 5,
+  kCyclePlainSplit = 6  // PLAIN on the split finest level (e0s, r32s)
 };
 constexpr size_t kMaxGraphs = 6;
 
@@ -1990,6 +2123,7 @@ pm_status enqueue_cycle(pm_mg* mg, int kind, float* phi, hipStream_t s) {
   Level& L0 = mg->lv[0];
   pm_status st;
   if (kind == kCyclePlain) return vcycle(mg, 0, s);
+  if (kind == kCyclePlainSplit) return vcycle_plain_split(mg, s);
   const bool fold_defect = kind == kCycleCarryFirstFold || kind == kCycleCarryMoreFold;
   const int carry = (kind == kCycleCarryFirst || kind == kCycleCarryFirstFold) ? kCarryFirst
                     : (kind == kCycleCarryMore || kind == kCycleCarryMoreFold) ? kCarryMore
@@ -2128,18 +2262,35 @@ pm_status solve_iterate(pm_mg* mg, float* phi, pm_mg_stats* stats, hipStream_t s
     double rhs_ss;
     if ((st = read_scalars(mg, mg->red + 3, 1, &rhs_ss, s))) return st;
     rhs_norm = std::sqrt(rhs_ss);
-    L0.phi = phi;
-    L0.rhs = mg->f0;
     mg->last_phi = phi;
+    // the cycles run on split copies of phi and f when phi can be read in quads
+    const bool split = mg->split_active() && mg->d.n_cycles > 0 &&
+                       (reinterpret_cast<uintptr_t>(phi) & 15u) == 0;
+    L0.phi = split ? mg->e0s : phi;
+    L0.rhs = split ? mg->r32s : mg->f0;
+    const int64_t quads = L0.nodes() / 8;
+    if (split) {
+      PM_TIMED("mg.to_split", 16.0 * L0.nodes(), s);
+      to_split4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(mg->f0, mg->r32s, L0.n, mg->hn);
+      PM_CHECK_LAUNCH("to_split4_kernel");
+      to_split4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(phi, mg->e0s, L0.n, mg->hn);
+      PM_CHECK_LAUNCH("to_split4_kernel");
+    }
     for (int c = 0; c < mg->d.n_cycles; ++c) {
-      if ((st = run_cycle(mg, kCyclePlain, phi, s))) return st;
+      if ((st = run_cycle(mg, split ? kCyclePlainSplit : kCyclePlain, split ? mg->e0s : phi, s)))
+        return st;
       if (c + 1 >= mg->d.min_cycles && rhs_norm > 0.0) {
-        if ((st = plain_residual_norm(mg, phi, &resid, s))) return st;
+        if ((st = plain_residual_norm(mg, phi, &resid, s, split))) return st;
         if (resid < mg->d.tol * rhs_norm) {
           cycles = c + 1;
           break;
         }
       }
+    }
+    if (split) {
+      PM_TIMED("mg.from_split", 8.0 * L0.nodes(), s);
+      from_split4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(mg->e0s, phi, L0.n, mg->hn);
+      PM_CHECK_LAUNCH("from_split4_kernel");
     }
   } else {
     const bool split = mg->split_active();
@@ -2199,6 +2350,13 @@ pm_status solve_iterate(pm_mg* mg, float* phi, pm_mg_stats* stats, hipStream_t s
   }
   return PM_OK;
 }
+
+// PLAIN grids from this size on (multiples of 8) run their cycles with the finest level in split
+// layout: a colour pass reads and writes half of what the natural one does (256^3 34 -> 18 us,
+// 128^3 7.5 -> 4.1; residual 36 -> 31, prolongation 52 -> 21), and the solve pays three copies
+// for it (21 us at 128^3). A cold 256^3 solve of 20 cycles 11.8 -> 8.5 ms; one warm cycle at
+// 128^3 gains 9 us of a 400 us step. At 64^3 a pass is all latency (3.5 us either way).
+constexpr int kPlainSplitMin = 96;
 
 }  // namespace
 
@@ -2314,6 +2472,15 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
           return st;
         }
       }
+    }
+  }
+  if (d.mode == PM_MG_PLAIN && d.grid_size % 8 == 0 && d.grid_size >= kPlainSplitMin &&
+      mg->lv.size() > 1 && mg->bottom_from != 0 && d.post_sweeps >= 1) {
+    mg->hn = d.grid_size / 2;
+    if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->e0s), sizeof(float) * n0)) ||
+        (st = dalloc(mg, reinterpret_cast<void**>(&mg->r32s), sizeof(float) * n0))) {
+      destroy(mg);
+      return st;
     }
   }
   hipError_t he = hipHostMalloc(&mg->host, sizeof(double) * pm::kRedMaxQ, 0);
@@ -2496,6 +2663,8 @@ pm_status pm_mg_vcycle(pm_mg* mg, hipStream_t s) {
     double v[4];
     return mixed_correct(mg, mg->last_phi, v, s);
   }
+  mg->lv[0].phi = mg->last_phi;  // the natural arrays, wherever the solve's cycles ran
+  mg->lv[0].rhs = mg->f0;
   return vcycle(mg, 0, s);
 }
 

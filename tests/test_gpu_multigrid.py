@@ -387,3 +387,31 @@ def test_one_launch_legs_equal_colour_passes(device, mode, n, sweeps, bottom):
     """The V-cycle legs that run in one launch each (tile regions in LDS) give bitwise the phi
     and the cycle counts of the per-pass kernels, cold and warm."""
     test_small_level_fused_sweep_equals_colour_passes(device, mode, n, sweeps, bottom)
+
+
+@pytest.mark.parametrize("n,sweeps,shift", [(96, (2, 2), 0), (104, (1, 1), 0), (128, (0, 1), 0),
+                                            (160, (2, 1), 0), (256, (2, 2), 0),
+                                            (96, (2, 2), 1)])
+def test_plain_split_finest_equals_natural(device, n, sweeps, shift):
+    """PLAIN cycles on the split copies of phi and f (non-zero faces, halving levels) give
+    bitwise the natural layout's phi and cycle counts, cold, warm and through one more V-cycle;
+    a phi that is not 16-byte aligned (shift) keeps the natural layout."""
+    announce(f"plain split finest level n={n} sweeps={sweeps} shift={shift}")
+    from galaxy_collision_amd.solver.multigrid import MultigridPoissonSolver
+
+    dx = 40.0 / n
+    rho = _t(_gaussian_rho(n, dx, 3.0 * dx, 1.0, centre=(0.46 * n * dx, 0.52 * n * dx,
+                                                          0.5 * n * dx)), device)
+    out = []
+    for split in (True, False):
+        s = MultigridPoissonSolver(n, dx=dx, grav_constant=1.0, pre_sweeps=sweeps[0],
+                                   post_sweeps=sweeps[1], n_cycles=4, split_fine=split)
+        phi = torch.zeros(n ** 3 + 4, device=device)[shift:shift + n ** 3].view(n, n, n)
+        s.solve(rho, phi)
+        c0, r0 = s.last_cycles, s.residual_norm()
+        s.solve(rho * 1.01, phi, warm_start=True)
+        c1 = s.last_cycles
+        s._vcycle(0)
+        out.append((phi.clone(), c0, c1, r0))
+    assert torch.equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
