@@ -157,6 +157,8 @@ _SIGNATURES = {
     "pm_deposit_plan_set_mode": [_vp, _i32],
     "pm_deposit_last_timing": [_vp, ctypes.POINTER(_f)],
     "pm_grad": [_vp, _vp, _vp, _vp, _i32, _f, _vp],
+    "pm_gather_work_bytes": [_i64, _i32, ctypes.POINTER(_i64)],
+    "pm_gather_work": [_vp] * 9 + [_i64, _i32, _f, _vp, _vp],
     "pm_gather": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _f, _vp],
     "pm_kick": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _f, _vp],
     "pm_drift": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _f, _vp],

@@ -182,10 +182,17 @@ def potential_to_accel(phi, ax_g, ay_g, az_g, dx: float = 1.0) -> None:
 def gather_acceleration(parts, ax_g, ay_g, az_g, acc_x, acc_y, acc_z, dx: float = 1.0) -> None:
     """CIC-interpolate the node acceleration field to the particles."""
     n = _grid_n(ax_g)
-    nat.call("pm_gather", nat.ptr(as_tensor(parts.pos_x)), nat.ptr(as_tensor(parts.pos_y)),
+    work = None
+    if parts.n >= 1 << 19:  # fewer never need workspace
+        size = ctypes.c_int64()
+        nat.call("pm_gather_work_bytes", int(parts.n), n, ctypes.byref(size))
+        if size.value:  # from torch's allocator, so that it belongs to this call's stream
+            work = torch.empty(size.value // 4, dtype=torch.float32,
+                               device=as_tensor(ax_g).device)
+    nat.call("pm_gather_work", nat.ptr(as_tensor(parts.pos_x)), nat.ptr(as_tensor(parts.pos_y)),
              nat.ptr(as_tensor(parts.pos_z)), nat.ptr(as_tensor(ax_g)), nat.ptr(as_tensor(ay_g)),
              nat.ptr(as_tensor(az_g)), nat.ptr(as_tensor(acc_x)), nat.ptr(as_tensor(acc_y)),
-             nat.ptr(as_tensor(acc_z)), int(parts.n), n, float(dx), nat.stream())
+             nat.ptr(as_tensor(acc_z)), int(parts.n), n, float(dx), nat.ptr(work), nat.stream())
 
 
 __all__ = ["deposit_density", "deposit_keys", "gather_acceleration", "potential_to_accel",

@@ -257,6 +257,16 @@ pm_status pm_gather_kick_drift4_reorder(const int32_t* order, const pm_particle_
                                         float h_close, float h_open, float dt,
                                         uint32_t* keys_out, hipStream_t stream);
 
+/* pm_gather with workspace (work: pm_gather_work_bytes(n_particles, grid_size) bytes of device
+ * memory, 16-byte aligned; null or a size of 0 is pm_gather itself): when many particles lie
+ * scattered in memory (decided on the device from a sample) the field is interleaved per node
+ * first. Bitwise pm_gather. */
+pm_status pm_gather_work_bytes(int64_t n_particles, int32_t grid_size, int64_t* out);
+pm_status pm_gather_work(const float* pos_x, const float* pos_y, const float* pos_z,
+                         const float* gx, const float* gy, const float* gz, float* acc_x,
+                         float* acc_y, float* acc_z, int64_t n_particles, int32_t grid_size,
+                         float dx, void* work, hipStream_t stream);
+
 /* Fused gather then kick(h): bitwise the same as pm_gather followed by pm_kick
  * (the closing half of reference integrator.py:100-131 `kdk_step`). */
 pm_status pm_gather_kick(const float* pos_x, const float* pos_y, const float* pos_z,

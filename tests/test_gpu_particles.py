@@ -457,3 +457,41 @@ def test_chain_reorder_every(device):
     assert_bitwise(a.gid.to_numpy()[back], icr.gid.astype(np.int32), "gid by pid")
     np.testing.assert_allclose(a.positions()[back], plain.positions(), rtol=0, atol=1e-4)
     np.testing.assert_allclose(a.velocities()[back], plain.velocities(), rtol=0, atol=1e-3)
+
+
+@pytest.mark.parametrize("n,np_,order,shift", [
+    (64, (1 << 19) + 1, "random", 0),
+    (65, 1 << 19, "random", 0),       # odd grid: nodes not in whole quads
+    (64, 1 << 19, "random", 1),       # unaligned fields
+    (64, 1 << 19, "cells", 0),        # cell order: the component arrays are read
+    (64, (1 << 19) - 1, "random", 0)  # below the workspace's particle count
+])
+def test_gather_with_workspace_is_the_gather(device, n, np_, order, shift):
+    """The gather that may interleave the field first is bitwise pm_gather, corners outside the
+    box included, whichever way the sampled order sends it."""
+    from galaxy_collision_amd import _native as nat
+    from galaxy_collision_amd.data import ParticleState
+    from galaxy_collision_amd.deposit import gather_acceleration
+
+    announce(f"gather with workspace n={n} N={np_} {order} shift={shift}")
+    dx = 0.5
+    rng = np.random.default_rng(n + np_)
+    pos = rng.uniform(-1.5 * dx, (n + 0.5) * dx, (np_, 3)).astype(np.float32)
+    if order == "cells":
+        c = np.floor(pos / dx).astype(np.int64)
+        pos = pos[np.lexsort((c[:, 2], c[:, 1], c[:, 0]))]
+    pos[7] = np.nan
+    parts = ParticleState(np_)
+    parts.load(pos)
+    g = [torch.randn(n ** 3 + 4, device=device)[shift:shift + n ** 3].view(n, n, n)
+         for _ in range(3)]
+    acc = [[torch.full((np_,), 7.0, device=device) for _ in range(3)] for _ in range(2)]
+    gather_acceleration(parts, *g, *acc[0], dx)
+    nat.call("pm_gather", nat.ptr(parts.pos_x.tensor), nat.ptr(parts.pos_y.tensor),
+             nat.ptr(parts.pos_z.tensor), *(nat.ptr(t) for t in g), *(nat.ptr(t) for t in acc[1]),
+             np_, n, dx, nat.stream())
+    for a, b in zip(*acc):
+        assert torch.equal(a, b)
+    size = ctypes.c_int64()
+    nat.call("pm_gather_work_bytes", np_, n, ctypes.byref(size))
+    assert size.value == (16 * (n ** 3 + 1) if np_ >= 1 << 19 else 0)
