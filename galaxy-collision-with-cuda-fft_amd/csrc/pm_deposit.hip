@@ -75,9 +75,12 @@ __global__ void __launch_bounds__(256) key_kernel(
 // 2. stable LSD radix sort (reduce-then-scan; no inter-workgroup waiting)
 // ---------------------------------------------------------------------------------------
 // Per-tile digit histogram, stored digit-major: hist[d * tiles + tile].
+// ITEMS keys per lane: a tile is 256 * ITEMS keys.
+template <int ITEMS>
 __global__ void __launch_bounds__(256) radix_hist_kernel(const uint32_t* __restrict__ keys,
                                                          int64_t np, int tiles, int shift,
                                                          int bits, uint32_t* __restrict__ hist) {
+  constexpr int kTile = 256 * ITEMS;
   __shared__ uint32_t cnt[1 << kMaxDigitBits];
   const int buckets = 1 << bits;
   const uint32_t mask = static_cast<uint32_t>(buckets - 1);
@@ -194,11 +197,13 @@ __global__ void __launch_bounds__(256) radix_scan_kernel(uint32_t* __restrict__ 
 // Stable scatter of one tile. Lane l of wave w, round r holds tile position
 // w*64*kSortItems + r*64 + l, so (wave, round, lane) order is input order. A null vals_in
 // stands for the identity (the first pass sorts particle indices).
+template <int ITEMS>
 __global__ void __launch_bounds__(256) radix_scatter_kernel(
     const uint32_t* __restrict__ keys_in, const int32_t* __restrict__ vals_in,
     uint32_t* __restrict__ keys_out, int32_t* __restrict__ vals_out,
     const uint32_t* __restrict__ hist, const uint32_t* __restrict__ digit_tot, int64_t np,
     int tiles, int shift, int bits) {
+  constexpr int kTile = 256 * ITEMS, kSortItems = ITEMS;
   __shared__ uint32_t wave_cnt[kSortWaves][1 << kMaxDigitBits];
   __shared__ uint32_t tile_base[1 << kMaxDigitBits];
   const int lane = threadIdx.x & 63;
@@ -1001,19 +1006,26 @@ int plan_digits(uint64_t limit, int bits[4]) {
 }
 
 pm_status sort(const uint32_t* keys_in, uint32_t* const keys[2], int32_t* const vals[2],
-               uint32_t* hist, uint32_t* digit, int64_t np, int shift, const int* bits,
-               int passes, int* out, hipStream_t stream) {
+               uint32_t* hist, int64_t hist_cap, uint32_t* digit, int64_t np, int shift,
+               const int* bits, int passes, int* out, hipStream_t stream) {
   PM_REQUIRE(passes >= 1 && passes <= 4, "radix sort: 1 to 4 passes");
-  const int tiles = static_cast<int>(tiles_of(np));
+  // small sets take small tiles: with 4096 keys a tile, fewer workgroups than CUs would each
+  // rank 16 rounds of keys one after the other
+  const bool small = np <= kSmallSort && small_hist_words(np) <= hist_cap;
+  const int tiles = static_cast<int>(small ? (np + kSmallTile - 1) / kSmallTile : tiles_of(np));
   int src = 0;
   for (int s = 0; s < passes; ++s) {
     const int b = bits[s];
     PM_REQUIRE(b >= 1 && b <= kMaxDigitBits, "radix sort: digit width out of range");
     const int buckets = 1 << b;
     const uint32_t* kin = s == 0 ? keys_in : keys[src];
+    const int32_t* vin = s == 0 ? nullptr : vals[src];
     {
       PM_TIMED("deposit.radix_hist", 4.0 * np, stream);
-      radix_hist_kernel<<<tiles, 256, 0, stream>>>(kin, np, tiles, shift, b, hist);
+      if (small)
+        radix_hist_kernel<kSmallTile / 256><<<tiles, 256, 0, stream>>>(kin, np, tiles, shift, b, hist);
+      else
+        radix_hist_kernel<kSortItems><<<tiles, 256, 0, stream>>>(kin, np, tiles, shift, b, hist);
       PM_CHECK_LAUNCH("radix_hist_kernel");
     }
     {
@@ -1023,10 +1035,15 @@ pm_status sort(const uint32_t* keys_in, uint32_t* const keys[2], int32_t* const 
     }
     {
       // read key (+ index after the first pass), write key + index
-      PM_LAUNCH_TIMED("deposit.radix_scatter", (s == 0 ? 12.0 : 16.0) * np,
-                      radix_scatter_kernel, tiles, 256, 0, stream, kin,
-                      s == 0 ? nullptr : vals[src], keys[1 - src], vals[1 - src], hist, digit,
-                      np, tiles, shift, b);
+      const double bytes = (s == 0 ? 12.0 : 16.0) * np;
+      if (small)
+        PM_LAUNCH_TIMED("deposit.radix_scatter", bytes, radix_scatter_kernel<kSmallTile / 256>,
+                        tiles, 256, 0, stream, kin, vin, keys[1 - src], vals[1 - src], hist, digit,
+                        np, tiles, shift, b);
+      else
+        PM_LAUNCH_TIMED("deposit.radix_scatter", bytes, radix_scatter_kernel<kSortItems>, tiles,
+                        256, 0, stream, kin, vin, keys[1 - src], vals[1 - src], hist, digit, np,
+                        tiles, shift, b);
       PM_CHECK_LAUNCH("radix_scatter_kernel");
     }
     src = 1 - src;
@@ -1048,6 +1065,7 @@ struct pm_deposit_plan {
   uint32_t* keys[2] = {nullptr, nullptr};
   int32_t* vals[2] = {nullptr, nullptr};
   uint32_t* hist = nullptr;
+  int64_t hist_cap = 0;         // words of hist
   uint32_t* digit = nullptr;
   float* sums = nullptr;
   float* head = nullptr;
@@ -1111,6 +1129,7 @@ void init_plan_shape(pm_deposit_plan* p, int n, int64_t cap) {
   const int64_t m = static_cast<int64_t>(n) + 1;
   p->sentinel = static_cast<uint32_t>(m * m * m);
   p->passes = pm::radix::plan_digits(p->sentinel, p->digit_bits);
+  p->hist_cap = pm::radix::hist_words(cap);
 }
 
 // Calls f(buffer pointer, element count, name) for every sorted-mode scratch buffer of a
@@ -1120,7 +1139,6 @@ template <class F>
 pm_status for_each_buffer(pm_deposit_plan* p, F&& f) {
   const int64_t cap = p->cap;
   const int64_t m = static_cast<int64_t>(p->n) + 1;
-  const int64_t tiles = (cap + kTile - 1) / kTile;
   const int64_t chunks = (cap + kChunk - 1) / kChunk;
   const int64_t nbricks = nbricks_of(p->n);
   pm_status st = PM_OK;
@@ -1128,7 +1146,7 @@ pm_status for_each_buffer(pm_deposit_plan* p, F&& f) {
       (st = f(p->keys[1], cap, "hipMalloc keys")) ||
       (st = f(p->vals[0], cap, "hipMalloc vals")) ||
       (st = f(p->vals[1], cap, "hipMalloc vals")) ||
-      (st = f(p->hist, tiles << kMaxDigitBits, "hipMalloc hist")) ||
+      (st = f(p->hist, p->hist_cap, "hipMalloc hist")) ||
       (st = f(p->digit, int64_t(1) << kMaxDigitBits, "hipMalloc digit")) ||
       (st = f(p->sums, 8 * cap, "hipMalloc sums")) ||
       (st = f(p->head, 8 * chunks, "hipMalloc head")) ||
@@ -1159,6 +1177,9 @@ pm_status pm_deposit_plan_create(int32_t n, int64_t cap, pm_deposit_plan** out) 
              "pm_deposit_plan_create: max_particles must be in [1, 2^31)");
   auto* p = new pm_deposit_plan();
   init_plan_shape(p, n, cap);
+  // room for small tiles too (the no-allocation scratch keeps to the large ones)
+  p->hist_cap = std::max(p->hist_cap,
+                         pm::radix::small_hist_words(std::min(cap, pm::radix::kSmallSort)));
   pm_status st = for_each_buffer(p, [](auto*& ptr, int64_t count, const char* what) {
     return alloc(&ptr, count, what);
   });
@@ -1272,6 +1293,7 @@ pm::depbrick::SortBuffers sort_buffers(pm_deposit_plan* p) {
   sb.vals[0] = p->vals[0];
   sb.vals[1] = p->vals[1];
   sb.hist = p->hist;
+  sb.hist_cap = p->hist_cap;
   sb.digit = p->digit;
   return sb;
 }
@@ -1365,7 +1387,8 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
   int src = 0;
   {
     pm_status st = pm::radix::sort(keys_in ? keys_in : plan->keys[0], plan->keys, plan->vals,
-                                   plan->hist, plan->digit, np, 0, plan->digit_bits,
+                                   plan->hist, plan->hist_cap, plan->digit, np, 0,
+                                   plan->digit_bits,
                                    plan->passes, &src, stream);
     if (st != PM_OK) return st;
   }

@@ -13,11 +13,12 @@ pm_status create(int n, int64_t cap, State** out);
 void destroy(State* st);
 
 // Sort buffers borrowed from the deposit plan: keys[2], vals[2] of cap entries, hist of
-// radix::hist_words(cap) words, digit of 2^radix::kMaxDigitBits words.
+// hist_cap >= radix::hist_words(cap) words, digit of 2^radix::kMaxDigitBits words.
 struct SortBuffers {
   uint32_t* keys[2];
   int32_t* vals[2];
   uint32_t* hist;
+  int64_t hist_cap;
   uint32_t* digit;
 };
 

@@ -1250,7 +1250,7 @@ pm_status deposit(State* st, const SortBuffers& sb, const float* px, const float
       PM_CHECK_LAUNCH("brick_key_kernel");
     }
     int src = 0;
-    if ((e = pm::radix::sort(sb.keys[0], sb.keys, sb.vals, sb.hist, sb.digit, np, 0, st->bits,
+    if ((e = pm::radix::sort(sb.keys[0], sb.keys, sb.vals, sb.hist, sb.hist_cap, sb.digit, np, 0, st->bits,
                              st->passes, &src, s)))
       return e;
     {

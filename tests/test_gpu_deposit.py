@@ -312,3 +312,27 @@ def test_drift_keys_and_keyed_deposit(device):
 
 def _np_u32(t):
     return t.cpu().numpy().view(np.uint32)
+
+
+@pytest.mark.parametrize("np_", [1, 1023, 1024, 1025, 3 << 19, (3 << 19) + 1])
+def test_sort_tiles_keep_the_stable_order(device, np_):
+    """Small and large radix tiles (the line between them, partial last tiles) give the keys and
+    the stable permutation, with a plan sized for these particles and with a larger one."""
+    announce(f"radix tiles N={np_}")
+    from galaxy_collision_amd.data import ParticleState
+    from galaxy_collision_amd.deposit import DepositPlan
+
+    n, dx = 40, 1.0
+    rng = np.random.default_rng(np_)
+    pos = rng.normal(20.0, 9.0, (np_, 3)).astype(np.float32)
+    parts = ParticleState(np_)
+    parts.load(pos, None, np.full(np_, 1.0, np.float32))
+    rho = torch.empty((n,) * 3, device=device)
+    keys = torch.empty(np_, dtype=torch.int32, device=device)
+    perm = torch.empty(np_, dtype=torch.int32, device=device)
+    ref = O.cell_keys(pos, n, dx)
+    for cap in (np_, 2 * np_ + 5000):
+        plan = DepositPlan(n, cap)
+        plan.deposit(parts.pos_x, parts.pos_y, parts.pos_z, parts.mass, np_, dx, rho, keys, perm)
+        assert_bitwise(keys.cpu().numpy().view(np.uint32), ref, "cell keys")
+        assert_bitwise(perm.cpu().numpy(), O.stable_perm(ref), "stable permutation")
