@@ -1140,55 +1140,144 @@ __global__ void __launch_bounds__(256) rbs4_first_kernel(float* __restrict__ e,
   *reinterpret_cast<float4*>(e + plane + q.t0) = make_float4(out1[0], out1[1], out1[2], out1[3]);
 }
 
-// residual_s_kernel, 4 positions of both colours (8 consecutive natural nodes) per thread.
-__global__ void __launch_bounds__(256) residual_s4_kernel(const float* __restrict__ e,
-                                                          const float* __restrict__ r,
-                                                          float* __restrict__ res, int n,
-                                                          int hn, float inv_h2) {
+// residual_s_kernel and restrict_kernel in one pass, 4 positions of both colours (8 consecutive
+// natural nodes) per thread: the fine residual is only ever read by the restriction, so it
+// stays in LDS. A workgroup owns tj coarse rows and marches along i over ti coarse planes:
+// thread (row, quad) of the 2*tj + 1 fine rows carries e's planes i-1, i, i+1 in registers,
+// writes its residuals of plane i to LDS (even and odd k apart, so that the restriction's
+// stride-2 reads are contiguous), and each thread adds the plane's 9 terms to its (up to
+// kRROut) coarse sums. The weighted sum runs over planes 2I-1, 2I, 2I+1 in that order, so a
+// plane of odd i closes coarse plane I and opens I+1: every sum keeps restrict_kernel's order
+// and is bit for bit its result. PMRR_FIGURES
+constexpr int kRRThreads = 512;
+constexpr int kRRThreadsMax = 1024;  // rows of more than 64 quads (n > 512)
+constexpr int kRRBlocks = 512;       // two workgroups on each of 256 CUs (see residual_restrict)
+constexpr int kRROut = 2;            // coarse values per thread and plane
+template <int T>
+__global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) residual_restrict_s4_kernel(
+    const float* __restrict__ e, const float* __restrict__ r, float* __restrict__ rhs_c,
+    float* __restrict__ phi_c, int n, int hn, int nc, float inv_h2, int tj, int ti) {
+  __shared__ __attribute__((aligned(16))) float s_res[2][T * 8];
   const int hq = hn >> 2;
-  const uint32_t quads = static_cast<uint32_t>(n) * n * hq;
-  const int64_t u = pm::xcd_block() * blockDim.x + threadIdx.x;
-  if (u >= quads) return;
-  const Quad q = quad_idx(static_cast<uint32_t>(u), n, hq);
-  const uint32_t plane = static_cast<uint32_t>(n) * n * hn;
-  float out[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (q.i >= 1 && q.i <= n - 2 && q.j >= 1 && q.j <= n - 2) {
-    const uint32_t nh = static_cast<uint32_t>(n) * hn;
-    // both colours' loads issue before either colour is evaluated
-    float s[2][4];
+  const int rows = 2 * tj + 1;  // rows * hq <= T
+  const int jt = (nc + tj - 1) / tj;
+  const int blk = static_cast<int>(pm::xcd_block());
+  const int J0 = (blk % jt) * tj, I0 = (blk / jt) * ti;
+  const int I1 = I0 + ti < nc ? I0 + ti : nc;
+  const int lr = static_cast<int>(threadIdx.x) / hq;
+  const int kk0 = (static_cast<int>(threadIdx.x) - lr * hq) * 4;
+  const int j = 2 * J0 - 1 + lr;
+  const bool mine = lr < rows, row = mine && j >= 1 && j <= n - 2;
+  const uint32_t nh = static_cast<uint32_t>(n) * hn;
+  const uint32_t plane = static_cast<uint32_t>(n) * nh;
+  const uint32_t jk = static_cast<uint32_t>(row ? j : 1) * hn + (mine ? kk0 : 0);
+  // this thread's coarse outputs: LDS offset of fine (2J-1, K) and the flat (J, K), or none
+  int lo[kRROut];
+  bool in[kRROut], own[kRROut];
+  uint32_t dst[kRROut];
+  float acc[kRROut];
+#pragma unroll
+  for (int m = 0; m < kRROut; ++m) {
+    const int o = static_cast<int>(threadIdx.x) + m * T;
+    const int jl = o / nc, K = o - jl * nc, J = J0 + jl;
+    own[m] = jl < tj && J < nc;
+    in[m] = own[m] && J >= 1 && J <= nc - 2 && K >= 1 && K <= nc - 2;
+    lo[m] = in[m] ? 2 * jl * n + K : 1;  // (1: a place that can be read)
+    dst[m] = static_cast<uint32_t>(J) * nc + K;
+    acc[m] = 0.0f;
+  }
+  // (planes past the grid read a clamped one: only masked residuals take their values)
+  auto plane_quads = [&](int i, float4 (&v)[2]) {
+    const uint32_t t = static_cast<uint32_t>(min(max(i, 0), n - 1)) * nh + jk;
+    v[0] = ld4(e, t);
+    v[1] = ld4(e, plane + t);
+  };
+  float4 em[2], ec[2], ep[2];
+  const int f0 = 2 * I0 - 1, f1 = 2 * I1 - 1;  // fine planes f0..f1
+  plane_quads(f0 - 1, em);
+  plane_quads(f0, ec);
+  for (int f = f0; f <= f1; ++f) {
+    // last inner k of the row, below the first where the row holds none (a branch on it would
+    // let the compiler move loads behind it)
+    const int klast = row && f >= 1 && f <= n - 2 ? n - 2 : 0;
+    const uint32_t t0 = static_cast<uint32_t>(min(max(f, 1), n - 2)) * nh + jk;
     NbrQuad nb[2];
-    float4 ev[2], rv[2];
+    float4 rv[2];
+    plane_quads(f + 1, ep);
 #pragma unroll
     for (int color = 0; color < 2; ++color) {
-      const uint32_t own = static_cast<uint32_t>(color) * plane;
-      nb[color] = quad_nbr_load(e + (plane - own), q.t0, nh, static_cast<uint32_t>(hn),
-                                (q.i + q.j + color) & 1);
-      ev[color] = ld4(e, own + q.t0);
-      rv[color] = ld4(r, own + q.t0);
+      const float* eo = e + (color ? 0u : plane);
+      nb[color].c = ld4(eo, t0 + hn);
+      nb[color].d = ld4(eo, t0 - hn);
+      nb[color].edge = eo[((f + j + color) & 1) ? t0 + 4 : t0 - 1];
+      rv[color] = ld4(r, (color ? plane : 0u) + t0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int color = 0; color < 2; ++color) quad_nbr_sum(nb[color], (q.i + q.j + color) & 1, s[color]);
-    // every node is evaluated and the faces masked afterwards (a branch around the face
-    // terms would let the compiler move the loads only they use behind it)
+    __builtin_amdgcn_sched_barrier(0);  // all loads leave before any arithmetic
+    float* const sp = s_res[f & 1];
+    float out[2][4];  // [k parity][position]
+    float val[2][4];
 #pragma unroll
     for (int color = 0; color < 2; ++color) {
-      const int p = (q.i + q.j + color) & 1;
+      const int p = (f + j + color) & 1;
+      nb[color].a = ep[1 - color];
+      nb[color].b = em[1 - color];
+      nb[color].m = ec[1 - color];
+      float sum[4];
+      quad_nbr_sum(nb[color], p, sum);
 #pragma unroll
       for (int k4 = 0; k4 < 4; ++k4) {
-        const int k = 2 * (q.kk0 + k4) + p;
-        const float lap = (s[color][k4] - 6.0f * at4(ev[color], k4)) * inv_h2;
-        const float val = at4(rv[color], k4) - lap;
-        out[2 * k4 + p] = (k >= 1 && k <= n - 2) ? val : 0.0f;
+        const int k = 2 * (kk0 + k4) + p;
+        const float lap = (sum[k4] - 6.0f * at4(ec[color], k4)) * inv_h2;
+        const float v = at4(rv[color], k4) - lap;
+        val[color][k4] = (k >= 1 && k <= klast) ? v : 0.0f;
       }
     }
-  }
-  float* dst = res + (static_cast<int64_t>(q.i) * n + q.j) * n + 2 * q.kk0;
-  if (2 * q.kk0 + 8 <= n) {
-    *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
-    *reinterpret_cast<float4*>(dst + 4) = make_float4(out[4], out[5], out[6], out[7]);
-  } else {
-    for (int k = 0; k < 8 && 2 * q.kk0 + k < n; ++k) dst[k] = out[k];
+    const bool swap = (f + j) & 1;  // colour 0 holds the odd k
+#pragma unroll
+    for (int k4 = 0; k4 < 4; ++k4) {
+      out[0][k4] = swap ? val[1][k4] : val[0][k4];
+      out[1][k4] = swap ? val[0][k4] : val[1][k4];
+    }
+    if (mine) {
+      *reinterpret_cast<float4*>(sp + lr * n + kk0) =
+          make_float4(out[0][0], out[0][1], out[0][2], out[0][3]);
+      *reinterpret_cast<float4*>(sp + lr * n + hn + kk0) =
+          make_float4(out[1][0], out[1][1], out[1][2], out[1][3]);
+    }
+    // one barrier a plane: a buffer is written again two planes on, past the next barrier,
+    // which every thread reaches after its reads of this plane
+    __syncthreads();
+    const bool odd = f & 1;
+    const float wa = odd ? 1.0f : 2.0f;
+    const int I = f >> 1;  // odd f: the coarse plane it closes (f0 closes none of this tile's)
+#pragma unroll
+    for (int m = 0; m < kRROut; ++m) {
+      float t[9];
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        const float* q = sp + lo[m] + b * n;
+        const float wb = wa * (b == 1 ? 2.0f : 1.0f);
+        t[3 * b] = wb * q[hn - 1];          // k = 2K-1
+        t[3 * b + 1] = wb * 2.0f * q[0];    // k = 2K
+        t[3 * b + 2] = wb * q[hn];          // k = 2K+1
+      }
+#pragma unroll
+      for (int x = 0; x < 9; ++x) acc[m] += t[x];
+      if (odd) {
+        if (f > f0 && own[m]) {
+          const uint32_t c = static_cast<uint32_t>(I) * nc * nc + dst[m];
+          rhs_c[c] = (in[m] && I >= 1 && I <= nc - 2) ? acc[m] / 64.0f : 0.0f;
+          phi_c[c] = 0.0f;  // the coarse correction starts from zero
+        }
+        acc[m] = 0.0f;
+#pragma unroll
+        for (int x = 0; x < 9; ++x) acc[m] += t[x];
+      }
+    }
+    em[0] = ec[0];
+    em[1] = ec[1];
+    ec[0] = ep[0];
+    ec[1] = ep[1];
   }
 }
 
@@ -1927,6 +2016,30 @@ unsigned split_update_blocks(const pm_mg* mg, const float* phi, double** partial
   return pm::red_blocks(plane);
 }
 
+// Residual of the split finest level (n % 8 == 0) and its restriction to level C, whose phi is
+// cleared: residual_restrict_s4_kernel with as many fine rows as its threads cover, and ti
+// coarse planes a workgroup so that the launch is one round of resident workgroups (256^3:
+// 28 us; 33-35 with three quarters or twice as many, whose last wave is nearly empty, or half).
+pm_status residual_restrict(const float* e, const float* r, const Level& L, const Level& C, int hn,
+                            hipStream_t s) {
+  const int T = hn / 4 > 64 ? kRRThreadsMax : kRRThreads;
+  int tj = (T / (hn / 4) - 1) / 2;
+  while (tj > 1 && tj * C.n > kRROut * T) --tj;
+  const int jt = (C.n + tj - 1) / tj;
+  const int it = std::max(1, kRRBlocks / jt);
+  const int ti = std::max(2, (C.n + it - 1) / it);
+  const unsigned blocks = static_cast<unsigned>(jt) * static_cast<unsigned>((C.n + ti - 1) / ti);
+  PM_TIMED(level_name("mg.residual_restrict", L.n), 9.0 * L.nodes(), s);
+  if (T == kRRThreads)
+    residual_restrict_s4_kernel<kRRThreads><<<blocks, kRRThreads, 0, s>>>(
+        e, r, C.rhs, C.phi, L.n, hn, C.n, L.inv_h2, tj, ti);
+  else
+    residual_restrict_s4_kernel<kRRThreadsMax><<<blocks, kRRThreadsMax, 0, s>>>(
+        e, r, C.rhs, C.phi, L.n, hn, C.n, L.inv_h2, tj, ti);
+  PM_CHECK_LAUNCH("residual_restrict_s4_kernel");
+  return PM_OK;
+}
+
 // The finest level of the MIXED correction in split layout: e0s = V(r32s) from a zero
 // start (pre/post sweeps >= 1), then phi += e0s with the norms in partials.
 pm_status vcycle_split0(pm_mg* mg, float* phi, int carry, hipStream_t s) {
@@ -1964,17 +2077,15 @@ pm_status vcycle_split0(pm_mg* mg, float* phi, int carry, hipStream_t s) {
     }
     if ((st = pass(0, q == 0)) || (st = pass(1, false))) return st;
   }
-  {
-    PM_TIMED(level_name("mg.residual_s", n), kResidualBytes * nodes, s);
-    if (quad)
-      residual_s4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, L.res, n, hn,
-                                                                      L.inv_h2);
-    else
+  if (quad) {
+    if ((st = residual_restrict(e, r, L, C, hn, s))) return st;
+  } else {
+    {
+      PM_TIMED(level_name("mg.residual_s", n), kResidualBytes * nodes, s);
       residual_s_kernel<<<pm::blocks_for(L.nodes()), pm::kBlock, 0, s>>>(e, r, L.res, n, hn,
                                                                           L.inv_h2);
-    PM_CHECK_LAUNCH("residual_s_kernel");
-  }
-  {
+      PM_CHECK_LAUNCH("residual_s_kernel");
+    }
     PM_TIMED(level_name("mg.restrict", n), kRestrictBytes * nodes, s);
     restrict_kernel<<<pm::blocks_for(C.nodes()), pm::kBlock, 0, s>>>(L.res, C.rhs, C.phi, n,
                                                                       C.n);
@@ -2042,16 +2153,7 @@ pm_status vcycle_plain_split(pm_mg* mg, hipStream_t s) {
   };
   pm_status st;
   if ((st = sweeps(mg->d.pre_sweeps))) return st;
-  {
-    PM_TIMED(level_name("mg.residual_s", n), kResidualBytes * nodes, s);
-    residual_s4_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, L.res, n, hn, L.inv_h2);
-    PM_CHECK_LAUNCH("residual_s4_kernel");
-  }
-  {
-    PM_TIMED(level_name("mg.restrict", n), kRestrictBytes * nodes, s);
-    restrict_kernel<<<pm::blocks_for(C.nodes()), pm::kBlock, 0, s>>>(L.res, C.rhs, C.phi, n, C.n);
-    PM_CHECK_LAUNCH("restrict_kernel");
-  }
+  if ((st = residual_restrict(e, r, L, C, hn, s))) return st;
   if ((st = vcycle(mg, 1, s))) return st;
   {
     PM_TIMED(level_name("mg.prolong_s", n), 4.0 * nodes, s);
