@@ -819,8 +819,8 @@ __global__ void __launch_bounds__(256) update_kernel(float* __restrict__ phi,
 // ---------------------------------------------------------------------------------------
 // The correction e and the defect r of the finest level are internal to the solver, so they
 // are stored split by colour: node (i, j, k) of colour q = (i+j+k)&1 sits at
-//   q * plane + (i*n + j) * hn + (k >> 1),   hn = (n+1)/2, plane = n*n*hn
-// (odd n leaves one pad slot in half of the rows). Every neighbour of a node has the other
+//   q * plane + (i*n + j) * hn + (k >> 1),   plane = n*n*hn
+// with hn = (n+1)/2 rounded up to whole quads (pad slots hold zero). Every neighbour of a node has the other
 // colour, and (i+-1, j, k), (i, j+-1, k) sit at the same k>>1, so a colour pass reads half
 // of e and half of r, contiguously, instead of all of both. Each kernel below evaluates the
 // same float expressions in the same order as its natural-layout counterpart, so the
@@ -853,60 +853,6 @@ __device__ __forceinline__ float split_nbr_sum(const float* __restrict__ eo, int
   const int64_t row = t - kk;
   return eo[t + nh] + eo[t - nh] + eo[t + hn] + eo[t - hn] + eo[row + ((k + 1) >> 1)] +
          eo[row + ((k - 1) >> 1)];
-}
-
-// One colour pass (rb_pass_kernel's update); ZERO: every neighbour is zero.
-template <bool ZERO>
-__global__ void __launch_bounds__(256) rbs_kernel(float* __restrict__ e,
-                                                  const float* __restrict__ r, int n, int hn,
-                                                  float h2, int color) {
-  const int64_t plane = static_cast<int64_t>(n) * n * hn;
-  const int64_t t = pm::xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= plane) return;
-  const SplitIdx q = split_idx(t, n, hn);
-  const int k = 2 * q.kk + ((q.i + q.j + color) & 1);
-  if (q.i < 1 || q.i > n - 2 || q.j < 1 || q.j > n - 2 || k < 1 || k > n - 2) return;
-  const int64_t own = static_cast<int64_t>(color) * plane;
-  const float sum =
-      ZERO ? 0.0f
-           : split_nbr_sum(e + (plane - own), t, q.kk, k, static_cast<int64_t>(n) * hn, hn);
-  e[own + t] = (sum - h2 * r[own + t]) / 6.0f;
-}
-
-// residual_kernel from the split e and r into the natural-layout res.
-__global__ void __launch_bounds__(256) residual_s_kernel(const float* __restrict__ e,
-                                                         const float* __restrict__ r,
-                                                         float* __restrict__ res, int n,
-                                                         int hn, float inv_h2) {
-  const int64_t n2 = static_cast<int64_t>(n) * n;
-  const int64_t c = pm::xcd_block() * blockDim.x + threadIdx.x;
-  if (c >= n2 * n) return;
-  const pm::Idx3 q3 = pm::idx3(c, n);
-  const int i = q3.i, j = q3.j, k = q3.k;
-  float out = 0.0f;
-  if (i >= 1 && i <= n - 2 && j >= 1 && j <= n - 2 && k >= 1 && k <= n - 2) {
-    const int64_t plane = n2 * hn;
-    const int64_t own = static_cast<int64_t>((i + j + k) & 1) * plane;
-    const int64_t t = (static_cast<int64_t>(i) * n + j) * hn + (k >> 1);
-    const float sum = split_nbr_sum(e + (plane - own), t, k >> 1, k,
-                                    static_cast<int64_t>(n) * hn, hn);
-    const float lap = (sum - 6.0f * e[own + t]) * inv_h2;
-    out = r[own + t] - lap;
-  }
-  res[c] = out;
-}
-
-// prolong_add_kernel on the colour-1 nodes of the split e.
-__global__ void __launch_bounds__(256) prolong_s_kernel(const float* __restrict__ phi_c,
-                                                        float* __restrict__ e, int n, int hn,
-                                                        int nc) {
-  const int64_t plane = static_cast<int64_t>(n) * n * hn;
-  const int64_t t = pm::xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= plane) return;
-  const SplitIdx q = split_idx(t, n, hn);
-  const int k = 2 * q.kk + ((q.i + q.j + 1) & 1);
-  if (q.i < 1 || q.i > n - 2 || q.j < 1 || q.j > n - 2 || k < 1 || k > n - 2) return;
-  e[plane + t] = e[plane + t] + prolong_value(phi_c, nc, q.i, q.j, k);
 }
 
 // The last colour-1 pass fused with update_kernel: phi += e over every node (e = 0 on the
@@ -990,7 +936,7 @@ __global__ void __launch_bounds__(256) residual64_s_kernel(const float* __restri
   if (threadIdx.x == 0) partials[blockIdx.x * pm::kRedMaxQ] = v[0];
 }
 
-// --- 4-wide variants (n % 8 == 0): a thread owns positions kk0 .. kk0+3 of one row ------
+// --- 4-wide variants: a thread owns positions kk0 .. kk0+3 of one row -------------------
 // The index math runs once per 4 nodes and the loads are 16-byte vectors: the (i+-1) and
 // (j+-1) rows, the node's own row of the other colour (its k+-1 neighbours, plus one
 // scalar past either end) and the rhs. The per-node expressions are those of the scalar
@@ -1063,7 +1009,7 @@ __device__ __forceinline__ void quad_nbr_sums(const float* __restrict__ eo, uint
 }
 
 // FACES: the array's faces hold values (PLAIN's phi) and keep them; otherwise they are zero.
-template <bool ZERO, bool FACES = false>
+template <bool FACES = false>
 __global__ void __launch_bounds__(256) rbs4_kernel(float* __restrict__ e,
                                                    const float* __restrict__ r, int n, int hn,
                                                    float h2, int color) {
@@ -1076,17 +1022,15 @@ __global__ void __launch_bounds__(256) rbs4_kernel(float* __restrict__ e,
   const uint32_t plane = static_cast<uint32_t>(n) * n * hn;
   const uint32_t own = static_cast<uint32_t>(color) * plane;
   const int p = (q.i + q.j + color) & 1;
-  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  NbrQuad nb;
-  if (!ZERO)
-    nb = quad_nbr_load(e + (plane - own), q.t0, static_cast<uint32_t>(n) * hn,
-                       static_cast<uint32_t>(hn), p);
+  const NbrQuad nb = quad_nbr_load(e + (plane - own), q.t0, static_cast<uint32_t>(n) * hn,
+                                   static_cast<uint32_t>(hn), p);
   const float4 rr = ld4(r, own + q.t0);
   // a row's two end nodes are faces: one of them lies in this quad's first or last position
   const bool end = FACES && (q.kk0 == 0 || q.kk0 + 4 == hn);
   const float4 old = end ? ld4(e, own + q.t0) : make_float4(0.f, 0.f, 0.f, 0.f);
   __builtin_amdgcn_sched_barrier(0);  // all loads leave before any arithmetic
-  if (!ZERO) quad_nbr_sum(nb, p, s);
+  float s[4];
+  quad_nbr_sum(nb, p, s);
   float out[4];
 #pragma unroll
   for (int k4 = 0; k4 < 4; ++k4) {
@@ -1097,7 +1041,38 @@ __global__ void __launch_bounds__(256) rbs4_kernel(float* __restrict__ e,
   *reinterpret_cast<float4*>(e + own + q.t0) = make_float4(out[0], out[1], out[2], out[3]);
 }
 
-// The first sweep of a cycle's pre-smoothing in one pass: rbs4_kernel<true> on colour 0
+// The last colour-1 pass of a split coarse level: rbs4_kernel<false> on colour 1, with both
+// colours written to the natural phi that the finer level prolongs from (inner nodes; its faces
+// stay zero from allocation). e's own colour-1 values are left as they were.
+__global__ void __launch_bounds__(256) rbs4_last_kernel(const float* __restrict__ e,
+                                                        const float* __restrict__ r,
+                                                        float* __restrict__ phi, int n, int hn,
+                                                        float h2) {
+  const int hq = hn >> 2;
+  const uint32_t quads = static_cast<uint32_t>(n) * n * hq;
+  const int64_t u = pm::xcd_block() * blockDim.x + threadIdx.x;
+  if (u >= quads) return;
+  const Quad q = quad_idx(static_cast<uint32_t>(u), n, hq);
+  if (q.i < 1 || q.i > n - 2 || q.j < 1 || q.j > n - 2) return;
+  const uint32_t plane = static_cast<uint32_t>(n) * n * hn;
+  const int p1 = (q.i + q.j + 1) & 1;
+  const NbrQuad nb = quad_nbr_load(e, q.t0, static_cast<uint32_t>(n) * hn,
+                                   static_cast<uint32_t>(hn), p1);
+  const float4 rr = ld4(r, plane + q.t0);
+  __builtin_amdgcn_sched_barrier(0);  // all loads leave before any arithmetic
+  float s[4];
+  quad_nbr_sum(nb, p1, s);
+  float* dst = phi + (static_cast<int64_t>(q.i) * n + q.j) * n + 2 * q.kk0;
+#pragma unroll
+  for (int k4 = 0; k4 < 4; ++k4) {
+    const float v1 = (s[k4] - h2 * at4(rr, k4)) / 6.0f, v0 = at4(nb.m, k4);
+    const int k = 2 * (q.kk0 + k4);
+    if (k >= 1 && k <= n - 2) dst[2 * k4] = p1 ? v0 : v1;
+    if (k + 1 <= n - 2) dst[2 * k4 + 1] = p1 ? v1 : v0;
+  }
+}
+
+// The first sweep of a cycle's pre-smoothing in one pass: colour 0
 // (zero guess: e0 = (0 - h2*r0)/6, 0 on faces) then rbs4_kernel<false> on colour 1, whose
 // colour-0 neighbours are those same values, computed here from r0 instead of read back
 // (r is 0 on faces and pad slots, so they come out 0 as written). Bitwise the two passes.
@@ -1148,7 +1123,12 @@ __global__ void __launch_bounds__(256) rbs4_first_kernel(float* __restrict__ e,
 // stride-2 reads are contiguous), and each thread adds the plane's 9 terms to its (up to
 // kRROut) coarse sums. The weighted sum runs over planes 2I-1, 2I, 2I+1 in that order, so a
 // plane of odd i closes coarse plane I and opens I+1: every sum keeps restrict_kernel's order
-// and is bit for bit its result. PMRR_FIGURES
+// and is bit for bit its result. hc > 0: the coarse level is split too (rows of hc positions)
+// and starts from zero without a cleared phi.
+// Memory bound: e and r are read once (134 MB at 256^3) and the coarse level written; the
+// separate passes also wrote and read the residual (another 134 MB): 42 + 18 us -> 30 in a
+// leapfrog step, 31 + 18 -> 28 in a cold solve. Every load of a plane leaves before its
+// arithmetic (97 registers; left to itself the compiler held loads back to stay at 64: 45 us).
 constexpr int kRRThreads = 512;
 constexpr int kRRThreadsMax = 1024;  // rows of more than 64 quads (n > 512)
 constexpr int kRRBlocks = 512;       // two workgroups on each of 256 CUs (see residual_restrict)
@@ -1156,9 +1136,10 @@ constexpr int kRROut = 2;            // coarse values per thread and plane
 template <int T>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) residual_restrict_s4_kernel(
     const float* __restrict__ e, const float* __restrict__ r, float* __restrict__ rhs_c,
-    float* __restrict__ phi_c, int n, int hn, int nc, float inv_h2, int tj, int ti) {
+    float* __restrict__ phi_c, int n, int hn, int nc, int hc, float inv_h2, int tj, int ti) {
   __shared__ __attribute__((aligned(16))) float s_res[2][T * 8];
   const int hq = hn >> 2;
+  const int ns = 2 * hn;        // LDS floats per fine row
   const int rows = 2 * tj + 1;  // rows * hq <= T
   const int jt = (nc + tj - 1) / tj;
   const int blk = static_cast<int>(pm::xcd_block());
@@ -1171,19 +1152,23 @@ __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) 
   const uint32_t nh = static_cast<uint32_t>(n) * hn;
   const uint32_t plane = static_cast<uint32_t>(n) * nh;
   const uint32_t jk = static_cast<uint32_t>(row ? j : 1) * hn + (mine ? kk0 : 0);
-  // this thread's coarse outputs: LDS offset of fine (2J-1, K) and the flat (J, K), or none
+  // this thread's coarse outputs: LDS offset of fine (2J-1, K) and the place of (0, J, K) in
+  // rhs_c, or none
   int lo[kRROut];
   bool in[kRROut], own[kRROut];
-  uint32_t dst[kRROut];
+  uint32_t dst[kRROut], par[kRROut];
   float acc[kRROut];
+  const uint32_t stride_c = static_cast<uint32_t>(nc) * (hc ? hc : nc);
+  const uint32_t plane_c = hc ? static_cast<uint32_t>(nc) * stride_c : 0u;
 #pragma unroll
   for (int m = 0; m < kRROut; ++m) {
     const int o = static_cast<int>(threadIdx.x) + m * T;
     const int jl = o / nc, K = o - jl * nc, J = J0 + jl;
     own[m] = jl < tj && J < nc;
     in[m] = own[m] && J >= 1 && J <= nc - 2 && K >= 1 && K <= nc - 2;
-    lo[m] = in[m] ? 2 * jl * n + K : 1;  // (1: a place that can be read)
-    dst[m] = static_cast<uint32_t>(J) * nc + K;
+    lo[m] = in[m] ? 2 * jl * ns + K : 1;  // (1: a place that can be read)
+    dst[m] = static_cast<uint32_t>(J) * (hc ? hc : nc) + (hc ? K >> 1 : K);
+    par[m] = static_cast<uint32_t>(J + K) & 1u;
     acc[m] = 0.0f;
   }
   // (planes past the grid read a clamped one: only masked residuals take their values)
@@ -1239,9 +1224,9 @@ __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       out[1][k4] = swap ? val[0][k4] : val[1][k4];
     }
     if (mine) {
-      *reinterpret_cast<float4*>(sp + lr * n + kk0) =
+      *reinterpret_cast<float4*>(sp + lr * ns + kk0) =
           make_float4(out[0][0], out[0][1], out[0][2], out[0][3]);
-      *reinterpret_cast<float4*>(sp + lr * n + hn + kk0) =
+      *reinterpret_cast<float4*>(sp + lr * ns + hn + kk0) =
           make_float4(out[1][0], out[1][1], out[1][2], out[1][3]);
     }
     // one barrier a plane: a buffer is written again two planes on, past the next barrier,
@@ -1255,7 +1240,7 @@ __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       float t[9];
 #pragma unroll
       for (int b = 0; b < 3; ++b) {
-        const float* q = sp + lo[m] + b * n;
+        const float* q = sp + lo[m] + b * ns;
         const float wb = wa * (b == 1 ? 2.0f : 1.0f);
         t[3 * b] = wb * q[hn - 1];          // k = 2K-1
         t[3 * b + 1] = wb * 2.0f * q[0];    // k = 2K
@@ -1265,9 +1250,10 @@ __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       for (int x = 0; x < 9; ++x) acc[m] += t[x];
       if (odd) {
         if (f > f0 && own[m]) {
-          const uint32_t c = static_cast<uint32_t>(I) * nc * nc + dst[m];
+          const uint32_t c = static_cast<uint32_t>(I) * stride_c + dst[m] +
+                             (((par[m] + I) & 1u) ? plane_c : 0u);
           rhs_c[c] = (in[m] && I >= 1 && I <= nc - 2) ? acc[m] / 64.0f : 0.0f;
-          phi_c[c] = 0.0f;  // the coarse correction starts from zero
+          if (!hc) phi_c[c] = 0.0f;  // the coarse correction starts from zero
         }
         acc[m] = 0.0f;
 #pragma unroll
@@ -1294,6 +1280,7 @@ constexpr int kProlongBlock = 256;  // threads of a prolong_s4_kernel workgroup
 constexpr int kProlongStageIt = (kProlongMaxLds + kProlongBlock - 1) / kProlongBlock;
 static_assert(kProlongBlock == pm::kBlock, "prolong_s4_kernel is launched with pm::kBlock");
 
+template <bool PAD>
 __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* __restrict__ phi_c,
                                                          float* __restrict__ e, int n, int hn,
                                                          int nc) {
@@ -1361,6 +1348,8 @@ __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* 
     // the fifth coarse value serves odd k; on a halving level the last quad's lies past the row
     // (only the face k = n - 1 would take it)
     const bool fifth = p && qq.kk0 + 4 < nc;
+    // PAD: the last quad's pad positions lie past the coarse row as well
+    auto has = [&](int x) { return (x < 4 || fifth) && (!PAD || qq.kk0 + x < nc); };
     float c[2][2][5];
 #pragma unroll
     for (int di = 0; di < 2; ++di) {
@@ -1371,12 +1360,12 @@ __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* 
           const int row = ((ci + di - ci0) * ncj + (cj + dj - cj0)) * nc + qq.kk0;
 #pragma unroll
           for (int x = 0; x < 5; ++x)
-            c[di][dj][x] = (need && (x < 4 || fifth)) ? s_c[row + x] : 0.0f;
+            c[di][dj][x] = (need && has(x)) ? s_c[row + x] : 0.0f;
         } else {
           const uint32_t row = (ci + di) * nc2 + static_cast<uint32_t>(cj + dj) * nc + qq.kk0;
 #pragma unroll
           for (int x = 0; x < 5; ++x)
-            c[di][dj][x] = (need && (x < 4 || fifth)) ? phi_c[row + x] : 0.0f;
+            c[di][dj][x] = (need && has(x)) ? phi_c[row + x] : 0.0f;
         }
       }
     }
@@ -1672,6 +1661,9 @@ struct Level {
   float* rhs = nullptr;  // level 0: 4*pi*G*rho (PLAIN) or the float32 defect (MIXED)
   float* res = nullptr;
   float* tmp = nullptr;  // ping-pong partner of phi for the fused sweep (large levels only)
+  float* es = nullptr;   // coarse levels swept in split layout: phi and rhs (zero faces and pads)
+  float* rs = nullptr;
+  int hs = 0;            // their row length
   int64_t nodes() const { return static_cast<int64_t>(n) * n * n; }
 };
 
@@ -1960,11 +1952,15 @@ pm_status leg_up(const Level& L, const Level& C, int sweeps, hipStream_t s) {
   return PM_OK;
 }
 
-pm_status vcycle(pm_mg* mg, size_t l, hipStream_t s) {
+pm_status vcycle_split(pm_mg* mg, size_t l, hipStream_t s);
+
+// split: called from a level in split layout, which wrote this level's rhs into rs if it has one.
+pm_status vcycle(pm_mg* mg, size_t l, hipStream_t s, bool split = false) {
   const Level& L = mg->lv[l];
   if (mg->use_bottom && mg->bottom_from >= 0 && static_cast<int>(l) >= mg->bottom_from)
     return bottom(mg, l, s);
   if (l + 1 == mg->lv.size()) return coarsest(mg, L, s);
+  if (split && L.es) return vcycle_split(mg, l, s);
   pm_status st;
   if (use_legs(mg, l)) {
     const Level& C = mg->lv[l + 1];
@@ -2016,14 +2012,17 @@ unsigned split_update_blocks(const pm_mg* mg, const float* phi, double** partial
   return pm::red_blocks(plane);
 }
 
-// Residual of the split finest level (n % 8 == 0) and its restriction to level C, whose phi is
-// cleared: residual_restrict_s4_kernel with as many fine rows as its threads cover, and ti
+// Row length of the split layout of an n^3 level: whole quads of positions.
+int split_row(int n) { return ((n + 1) / 2 + 3) / 4 * 4; }
+
+// Residual of a split level L and its restriction to level C (its split rhs, or its natural one
+// with phi cleared): residual_restrict_s4_kernel with as many fine rows as its threads cover, and ti
 // coarse planes a workgroup so that the launch is one round of resident workgroups (256^3:
 // 28 us; 33-35 with three quarters or twice as many, whose last wave is nearly empty, or half).
 pm_status residual_restrict(const float* e, const float* r, const Level& L, const Level& C, int hn,
                             hipStream_t s) {
   const int T = hn / 4 > 64 ? kRRThreadsMax : kRRThreads;
-  int tj = (T / (hn / 4) - 1) / 2;
+  int tj = std::min((T / (hn / 4) - 1) / 2, C.n);
   while (tj > 1 && tj * C.n > kRROut * T) --tj;
   const int jt = (C.n + tj - 1) / tj;
   const int it = std::max(1, kRRBlocks / jt);
@@ -2032,11 +2031,72 @@ pm_status residual_restrict(const float* e, const float* r, const Level& L, cons
   PM_TIMED(level_name("mg.residual_restrict", L.n), 9.0 * L.nodes(), s);
   if (T == kRRThreads)
     residual_restrict_s4_kernel<kRRThreads><<<blocks, kRRThreads, 0, s>>>(
-        e, r, C.rhs, C.phi, L.n, hn, C.n, L.inv_h2, tj, ti);
+        e, r, C.es ? C.rs : C.rhs, C.phi, L.n, hn, C.n, C.hs, L.inv_h2, tj, ti);
   else
     residual_restrict_s4_kernel<kRRThreadsMax><<<blocks, kRRThreadsMax, 0, s>>>(
-        e, r, C.rhs, C.phi, L.n, hn, C.n, L.inv_h2, tj, ti);
+        e, r, C.es ? C.rs : C.rhs, C.phi, L.n, hn, C.n, C.hs, L.inv_h2, tj, ti);
   PM_CHECK_LAUNCH("residual_restrict_s4_kernel");
+  return PM_OK;
+}
+
+pm_status prolong_split(const Level& C, float* e, int n, int hn, hipStream_t s) {
+  const int64_t quads = static_cast<int64_t>(n) * n * hn / 4;
+  const unsigned blocks = pm::blocks_for((quads + kProlongQ - 1) / kProlongQ);
+  PM_TIMED(level_name("mg.prolong_s", n), 4.0 * n * n * n, s);
+  if (n % 8 == 0)
+    prolong_s4_kernel<false><<<blocks, pm::kBlock, 0, s>>>(C.phi, e, n, hn, C.n);
+  else
+    prolong_s4_kernel<true><<<blocks, pm::kBlock, 0, s>>>(C.phi, e, n, hn, C.n);
+  PM_CHECK_LAUNCH("prolong_s4_kernel");
+  return PM_OK;
+}
+
+// Smoothing of a split level that starts from zero (`count` >= 1 sweeps, the first in one pass).
+pm_status smooth_from_zero(float* e, const float* r, const Level& L, int hn, int count,
+                           hipStream_t s) {
+  const int64_t quads = static_cast<int64_t>(L.n) * L.n * hn / 4;
+  const unsigned blocks = pm::blocks_for(quads);
+  const double nodes = static_cast<double>(L.nodes());
+  for (int q = 0; q < count; ++q) {
+    PM_TIMED(level_name(q ? "mg.rbs" : "mg.rbs_first", L.n), (q ? 12.0 : 8.0) * nodes, s);
+    if (q == 0) {
+      rbs4_first_kernel<<<blocks, pm::kBlock, 0, s>>>(e, r, L.n, hn, L.h2);
+    } else {
+      rbs4_kernel<false><<<blocks, pm::kBlock, 0, s>>>(e, r, L.n, hn, L.h2, 0);
+      rbs4_kernel<false><<<blocks, pm::kBlock, 0, s>>>(e, r, L.n, hn, L.h2, 1);
+    }
+    PM_CHECK_LAUNCH("rbs4_kernel");
+  }
+  return PM_OK;
+}
+
+// Post-smoothing of a split level up to its last colour-1 pass, which the caller fuses with
+// what it does with the result.
+pm_status smooth_before_last(float* e, const float* r, const Level& L, int hn, int count,
+                             hipStream_t s) {
+  const unsigned blocks = pm::blocks_for(static_cast<int64_t>(L.n) * L.n * hn / 4);
+  for (int q = 0; q < 2 * count - 1; ++q) {
+    PM_TIMED(level_name("mg.rbs", L.n), 6.0 * L.nodes(), s);
+    rbs4_kernel<false><<<blocks, pm::kBlock, 0, s>>>(e, r, L.n, hn, L.h2, q & 1);
+    PM_CHECK_LAUNCH("rbs4_kernel");
+  }
+  return PM_OK;
+}
+
+// A coarse level in split layout: L.phi = V(rs) from a zero start (pre/post sweeps >= 1).
+pm_status vcycle_split(pm_mg* mg, size_t l, hipStream_t s) {
+  const Level& L = mg->lv[l];
+  const Level& C = mg->lv[l + 1];
+  pm_status st;
+  if ((st = smooth_from_zero(L.es, L.rs, L, L.hs, mg->d.pre_sweeps, s)) ||
+      (st = residual_restrict(L.es, L.rs, L, C, L.hs, s)) || (st = vcycle(mg, l + 1, s, true)) ||
+      (st = prolong_split(C, L.es, L.n, L.hs, s)) ||
+      (st = smooth_before_last(L.es, L.rs, L, L.hs, mg->d.post_sweeps, s)))
+    return st;
+  PM_TIMED(level_name("mg.rbs_last", L.n), 10.0 * L.nodes(), s);
+  rbs4_last_kernel<<<pm::blocks_for(static_cast<int64_t>(L.n) * L.n * L.hs / 4), pm::kBlock, 0,
+                     s>>>(L.es, L.rs, L.phi, L.n, L.hs, L.h2);
+  PM_CHECK_LAUNCH("rbs4_last_kernel");
   return PM_OK;
 }
 
@@ -2046,72 +2106,23 @@ pm_status vcycle_split0(pm_mg* mg, float* phi, int carry, hipStream_t s) {
   const Level& L = mg->lv[0];
   const Level& C = mg->lv[1];
   const int n = L.n, hn = mg->hn;
-  const int64_t plane = static_cast<int64_t>(n) * n * hn;
   const double nodes = static_cast<double>(L.nodes());
   float* e = mg->e0s;
   const float* r = mg->r32s;
-  // 4 positions per thread when rows split into aligned quads (n % 8 == 0)
-  const bool quad = n % 8 == 0;
-  const bool phi_aligned = (reinterpret_cast<uintptr_t>(phi) & 15u) == 0;
-  const int64_t quads = plane / 4;
-  auto pass = [&](int color, bool zero) -> pm_status {
-    PM_TIMED(level_name(zero ? "mg.rbs0" : "mg.rbs", n), (zero ? 4.0 : 6.0) * nodes, s);
-    if (quad && zero)
-      rbs4_kernel<true><<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, color);
-    else if (quad)
-      rbs4_kernel<false><<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, color);
-    else if (zero)
-      rbs_kernel<true><<<pm::blocks_for(plane), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, color);
-    else
-      rbs_kernel<false><<<pm::blocks_for(plane), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, color);
-    PM_CHECK_LAUNCH("rbs_kernel");
-    return PM_OK;
-  };
   pm_status st;
-  for (int q = 0; q < mg->d.pre_sweeps; ++q) {
-    if (q == 0 && quad) {  // zero-guess colour 0 and colour 1 in one pass
-      PM_TIMED(level_name("mg.rbs_first", n), 8.0 * nodes, s);
-      rbs4_first_kernel<<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2);
-      PM_CHECK_LAUNCH("rbs4_first_kernel");
-      continue;
-    }
-    if ((st = pass(0, q == 0)) || (st = pass(1, false))) return st;
-  }
-  if (quad) {
-    if ((st = residual_restrict(e, r, L, C, hn, s))) return st;
-  } else {
-    {
-      PM_TIMED(level_name("mg.residual_s", n), kResidualBytes * nodes, s);
-      residual_s_kernel<<<pm::blocks_for(L.nodes()), pm::kBlock, 0, s>>>(e, r, L.res, n, hn,
-                                                                          L.inv_h2);
-      PM_CHECK_LAUNCH("residual_s_kernel");
-    }
-    PM_TIMED(level_name("mg.restrict", n), kRestrictBytes * nodes, s);
-    restrict_kernel<<<pm::blocks_for(C.nodes()), pm::kBlock, 0, s>>>(L.res, C.rhs, C.phi, n,
-                                                                      C.n);
-    PM_CHECK_LAUNCH("restrict_kernel");
-  }
-  if ((st = vcycle(mg, 1, s))) return st;
-  {
-    PM_TIMED(level_name("mg.prolong_s", n), 4.0 * nodes, s);
-    if (quad)
-      prolong_s4_kernel<<<pm::blocks_for((quads + kProlongQ - 1) / kProlongQ), pm::kBlock, 0,
-                          s>>>(C.phi, e, n, hn, C.n);
-    else
-      prolong_s_kernel<<<pm::blocks_for(plane), pm::kBlock, 0, s>>>(C.phi, e, n, hn, C.n);
-    PM_CHECK_LAUNCH("prolong_s_kernel");
-  }
-  for (int q = 0; q < mg->d.post_sweeps; ++q) {
-    if ((st = pass(0, false))) return st;
-    if (q + 1 < mg->d.post_sweeps && (st = pass(1, false))) return st;
-  }
+  if ((st = smooth_from_zero(e, r, L, hn, mg->d.pre_sweeps, s)) ||
+      (st = residual_restrict(e, r, L, C, hn, s)) || (st = vcycle(mg, 1, s, true)) ||
+      (st = prolong_split(C, e, n, hn, s)) ||
+      (st = smooth_before_last(e, r, L, hn, mg->d.post_sweeps, s)))
+    return st;
   {
     PM_TIMED("mg.black_update", (carry != kCarryNone ? 20.0 : 12.0) * nodes, s);
     double* partials;
     const unsigned blocks = split_update_blocks(mg, phi, &partials);
     float* g = mg->guess;
-    const bool vec = quad && phi_aligned && (carry == kCarryNone ||
-                                             (reinterpret_cast<uintptr_t>(g) & 15u) == 0);
+    // 8 natural nodes per thread when phi's rows are whole quads (n % 8 == 0)
+    auto aligned = [](const float* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    const bool vec = n % 8 == 0 && aligned(phi) && (carry == kCarryNone || aligned(g));
 #define PM_BLACK_UPDATE(K, C)                                                        \
   K<C><<<blocks, pm::kBlock, 0, s>>>(e, r, phi, g, n, hn, L.h2, partials)
     if (vec && carry == kCarryFirst)
@@ -2146,7 +2157,7 @@ pm_status vcycle_plain_split(pm_mg* mg, hipStream_t s) {
   auto sweeps = [&](int count) -> pm_status {
     for (int q = 0; q < 2 * count; ++q) {
       PM_TIMED(level_name("mg.rbs", n), 6.0 * nodes, s);
-      rbs4_kernel<false, true><<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, q & 1);
+      rbs4_kernel<true><<<pm::blocks_for(quads), pm::kBlock, 0, s>>>(e, r, n, hn, L.h2, q & 1);
       PM_CHECK_LAUNCH("rbs4_kernel");
     }
     return PM_OK;
@@ -2154,13 +2165,7 @@ pm_status vcycle_plain_split(pm_mg* mg, hipStream_t s) {
   pm_status st;
   if ((st = sweeps(mg->d.pre_sweeps))) return st;
   if ((st = residual_restrict(e, r, L, C, hn, s))) return st;
-  if ((st = vcycle(mg, 1, s))) return st;
-  {
-    PM_TIMED(level_name("mg.prolong_s", n), 4.0 * nodes, s);
-    prolong_s4_kernel<<<pm::blocks_for((quads + kProlongQ - 1) / kProlongQ), pm::kBlock, 0, s>>>(
-        C.phi, e, n, hn, C.n);
-    PM_CHECK_LAUNCH("prolong_s4_kernel");
-  }
+  if ((st = vcycle(mg, 1, s, true)) || (st = prolong_split(C, e, n, hn, s))) return st;
   return sweeps(mg->d.post_sweeps);
 }
 
@@ -2577,7 +2582,7 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
     }
     if (mg->lv.size() > 1 && mg->bottom_from != 0 && d.pre_sweeps >= 1 && d.post_sweeps >= 1) {
       const int n = mg->lv[0].n;
-      mg->hn = (n + 1) / 2;
+      mg->hn = split_row(n);
       const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(n) * n * mg->hn;
       if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->e0s), bytes)) ||
           (st = dalloc(mg, reinterpret_cast<void**>(&mg->r32s), bytes))) {
@@ -2614,6 +2619,27 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
         (st = dalloc(mg, reinterpret_cast<void**>(&mg->r32s), sizeof(float) * n0))) {
       destroy(mg);
       return st;
+    }
+  }
+  // coarse levels below a split one, down to the sizes that one launch per leg or sweep serves
+  if (mg->e0s && d.pre_sweeps >= 1 && d.post_sweeps >= 1) {
+    for (size_t l = 1; l + 1 < mg->lv.size(); ++l) {
+      Level& L = mg->lv[l];
+      if (L.n <= kLegMax || (mg->bottom_from >= 0 && static_cast<int>(l) >= mg->bottom_from)) break;
+      L.hs = split_row(L.n);
+      const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(L.n) * L.n * L.hs;
+      for (float** q : {&L.es, &L.rs}) {
+        if ((st = dalloc(mg, reinterpret_cast<void**>(q), bytes))) {
+          destroy(mg);
+          return st;
+        }
+        hipError_t ze = hipMemset(*q, 0, bytes);
+        if (ze == hipSuccess) ze = hipDeviceSynchronize();
+        if (ze != hipSuccess) {
+          destroy(mg);
+          return pm::hip_fail("hipMemset (multigrid split levels)", ze);
+        }
+      }
     }
   }
   hipError_t he = hipHostMalloc(&mg->host, sizeof(double) * pm::kRedMaxQ, 0);

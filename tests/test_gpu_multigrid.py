@@ -439,3 +439,29 @@ def test_residual_and_restriction_in_one_pass(device, kind, n):
         out.append(phi)
     assert bool(torch.isfinite(out[0]).all())
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("kind,n,sweeps", [
+    ("mixed", 18, (1, 1)), ("mixed", 21, (2, 1)), ("mixed", 47, (1, 2)), ("mixed", 129, (1, 1)),
+    ("mixed", 145, (2, 2)), ("mixed", 256, (1, 3)), ("mixed", 321, (1, 1)),
+    ("plain", 144, (1, 1)), ("plain", 200, (2, 2)), ("plain", 256, (0, 1)), ("plain", 304, (3, 1))])
+def test_split_levels_equal_natural_levels(device, kind, n, sweeps):
+    """Split finest grids of any size (rows that are not whole quads, few rows) and split coarse
+    levels (73, 129, 161 and 72, 100, 128, 152 nodes) against the natural layout: bitwise the
+    same phi after two cycles on a random density."""
+    announce(f"split levels {kind} n={n} sweeps={sweeps}")
+    from galaxy_collision_amd.solver.multigrid import (MixedPrecisionMultigridSolver,
+                                                       MultigridPoissonSolver)
+
+    cls = MixedPrecisionMultigridSolver if kind == "mixed" else MultigridPoissonSolver
+    g = torch.Generator().manual_seed(n)
+    rho = torch.rand((n, n, n), generator=g).to(device)
+    out = []
+    for split in (True, False):
+        s = cls(n, dx=40.0 / n, grav_constant=1.0, n_cycles=2, tol=1e-30, pre_sweeps=sweeps[0],
+                post_sweeps=sweeps[1], split_fine=split)
+        phi = torch.zeros((n, n, n), device=device)
+        s.solve(rho, phi)
+        out.append(phi)
+    assert bool(torch.isfinite(out[0]).all())
+    assert torch.equal(out[0], out[1])
