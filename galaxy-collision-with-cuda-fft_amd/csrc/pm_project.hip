@@ -30,32 +30,40 @@
 
 namespace {
 
-// bit pattern of the largest mass (masses are non-negative, so their float bits order like
-// the values); one atomic per workgroup
-__global__ void __launch_bounds__(256) max_mass_kernel(const float* __restrict__ mass, int64_t n,
-                                                       unsigned int* __restrict__ out) {
-  __shared__ unsigned int s[256];
+// Largest value over the workgroup (256 threads), in every thread. Uniform control flow only.
+__device__ __forceinline__ unsigned int block_max(unsigned int m) {
+  __shared__ unsigned int s[4];
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned int o = __shfl_xor(m, off, 64);
+    m = o > m ? o : m;
+  }
+  if ((threadIdx.x & 63u) == 0) s[threadIdx.x >> 6] = m;
+  __syncthreads();
+  for (int w = 0; w < 4; ++w) m = s[w] > m ? s[w] : m;
+  return m;
+}
+
+// First launch of the direct path: clears acc[0..cells] and leaves each workgroup's largest
+// mass (bit patterns: masses are non-negative, so their float bits order like the values) in
+// maxima[blockIdx.x]; the scatter's workgroups reduce those, so the maximum costs no launch of
+// its own (20,000 particles on 256 bins 15.6 us a frame with four launches, 14.2 with three;
+// 190,000 on 512 24.5 -> 16.1).
+constexpr int kMaxima = 1024;
+__global__ void __launch_bounds__(256) clear_max_kernel(const float* __restrict__ mass, int64_t n,
+                                                        unsigned long long* __restrict__ acc,
+                                                        int64_t cells,
+                                                        unsigned int* __restrict__ maxima) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
   unsigned int m = 0u;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+  for (int64_t i = t; i < n; i += step) {
     const float v = mass[i];
     const unsigned int b = v > 0.0f ? __float_as_uint(v) : 0u;
     m = b > m ? b : m;
   }
-  s[threadIdx.x] = m;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (static_cast<int>(threadIdx.x) < off && s[threadIdx.x + off] > s[threadIdx.x])
-      s[threadIdx.x] = s[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicMax(out, s[0]);
-}
-
-__global__ void __launch_bounds__(256) zero_u64_kernel(unsigned long long* __restrict__ p,
-                                                       int64_t count) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < count) p[i] = 0ull;
+  for (int64_t i = t; i <= cells; i += step) acc[i] = 0ull;
+  m = block_max(m);
+  if (threadIdx.x == 0) maxima[blockIdx.x] = m;
 }
 
 // scale exponent: largest mass * 2^s < 2^34 (s from the max mass's binary exponent)
@@ -90,14 +98,21 @@ __global__ void __launch_bounds__(256) project_kernel(const float* __restrict__ 
                                                       const float* __restrict__ mass, int64_t n,
                                                       float lo_a, float lo_b, float binw_a,
                                                       float binw_b, int bins,
-                                                      const unsigned int* __restrict__ maxbits,
+                                                      const unsigned int* __restrict__ maxima,
+                                                      int nmax,
+                                                      unsigned int* __restrict__ maxbits,
                                                       unsigned long long* __restrict__ acc) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int ia, ib;
-  if (!bin_of(pa[i], pb[i], lo_a, lo_b, binw_a, binw_b, bins, ia, ib)) return;
-  const unsigned long long q = fixed_mass(mass[i], *maxbits);
-  if (q) atomicAdd(&acc[static_cast<int64_t>(ia) * bins + ib], q);
+  unsigned int top = 0u;
+  for (int t = threadIdx.x; t < nmax; t += blockDim.x) top = maxima[t] > top ? maxima[t] : top;
+  top = block_max(top);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *maxbits = top;  // for unscale_kernel
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    int ia, ib;
+    if (!bin_of(pa[i], pb[i], lo_a, lo_b, binw_a, binw_b, bins, ia, ib)) continue;
+    const unsigned long long q = fixed_mass(mass[i], top);
+    if (q) atomicAdd(&acc[static_cast<int64_t>(ia) * bins + ib], q);
+  }
 }
 
 // ---- tiled path ------------------------------------------------------------------------
@@ -354,7 +369,7 @@ TiledLayout tiled_layout(int64_t n, int bins) {
 // The direct path's cost is the queue at the hottest bins, which shortens as the bins get
 // smaller; the tiled path costs 40-90 us up to a million particles, more of it the more tiles
 // a chunk touches. Measured on the collision's disks (direct / tiled, us): 65,536 particles on
-// 128 bins 60 / 42; 200,000 on 512 56 / 52, on 1024 42 / 83; 1,000,000 on 1024 154 / 74;
+// 128 bins 60 / 42; 200,000 on 512 53 / 53, on 1024 28 / 83; 1,000,000 on 1024 154 / 74;
 // 10,000,002 on 512 3447 / 119 in cell order, 1763 / 133 in random order. kMaxTiles bounds
 // the bins.
 bool use_tiled(int64_t n, int bins) {
@@ -390,13 +405,16 @@ pm_status pm_project_mass(const float* pos_a, const float* pos_b, const float* m
   auto* acc = static_cast<unsigned long long*>(scratch);
   auto* maxbits = reinterpret_cast<unsigned int*>(acc + cells);
   PM_TIMED("project", 16.0 * static_cast<double>(n) + 12.0 * static_cast<double>(cells), s);
-  zero_u64_kernel<<<pm::blocks_for(cells + 1), 256, 0, s>>>(acc, cells + 1);
-  PM_CHECK_LAUNCH("zero_u64_kernel");
+  // the workgroups' maxima lie in the image until unscale_kernel writes it
+  auto* maxima = reinterpret_cast<unsigned int*>(img);
+  const int nmax = static_cast<int>(
+      std::min({static_cast<int64_t>(pm::stream_blocks(std::max(n, cells + 1))), cells,
+                static_cast<int64_t>(kMaxima)}));
+  clear_max_kernel<<<static_cast<unsigned>(nmax), 256, 0, s>>>(mass, n, acc, cells, maxima);
+  PM_CHECK_LAUNCH("clear_max_kernel");
   if (n > 0) {
-    max_mass_kernel<<<pm::stream_blocks(n), 256, 0, s>>>(mass, n, maxbits);
-    PM_CHECK_LAUNCH("max_mass_kernel");
-    project_kernel<<<pm::blocks_for(n), 256, 0, s>>>(pos_a, pos_b, mass, n, lo_a, lo_b, binw_a,
-                                                     binw_b, bins, maxbits, acc);
+    project_kernel<<<pm::stream_blocks(n), 256, 0, s>>>(pos_a, pos_b, mass, n, lo_a, lo_b, binw_a,
+                                                        binw_b, bins, maxima, nmax, maxbits, acc);
     PM_CHECK_LAUNCH("project_kernel");
   }
   unscale_kernel<<<pm::blocks_for(cells), 256, 0, s>>>(acc, cells, maxbits, img);
