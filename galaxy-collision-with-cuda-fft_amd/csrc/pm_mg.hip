@@ -1399,7 +1399,9 @@ __global__ void __launch_bounds__(kProlongBlock) prolong_s4_kernel(const float* 
 // are the same; the squared norm is summed in another order. A thread takes kRes64Q such
 // runs (quads u, u + 256, ...) and issues the loads of all of them before any arithmetic
 // (2 measured slower than 1 at 256^3: 140 VGPRs halve the waves in flight).
+// SPLIT: r32s in split layout, else natural.
 constexpr int kRes64Q = 1;
+template <bool SPLIT>
 __global__ void __launch_bounds__(256) residual64_s4_kernel(const float* __restrict__ phi,
                                                             const float* __restrict__ rho,
                                                             float factor, int n,
@@ -1471,6 +1473,12 @@ __global__ void __launch_bounds__(256) residual64_s4_kernel(const float* __restr
           const double acc = v[0] + r * r;
           v[0] = inner ? acc : v[0];
         }
+      }
+      if (!SPLIT) {
+        float* dst = r32s + c0[m];
+        *reinterpret_cast<float4*>(dst) = make_float4(r8[0], r8[1], r8[2], r8[3]);
+        *reinterpret_cast<float4*>(dst + 4) = make_float4(r8[4], r8[5], r8[6], r8[7]);
+        continue;
       }
       // colour of natural k = 2*kk0 + x is (p0 + x) & 1; its position kk0 + (x >> 1)
       const int p0 = (q[m].i + q[m].j) & 1;
@@ -1698,7 +1706,7 @@ constexpr double kUpdBytes = 12.0;       // read phi + e, write phi
 struct pm_mg {
   pm_mg_desc d{};
   std::vector<Level> lv;
-  float* f0 = nullptr;        // 4*pi*G*rho, float32 (PLAIN, and the network's input)
+  float* f0 = nullptr;        // 4*pi*G*rho, float32 (PLAIN)
   const float* cur_rho = nullptr;  // rho of the last setup (the float64 defect scales it)
   float factor = 0.0f;             // 4*pi*G as float32
   float* e0 = nullptr;        // MIXED: finest correction
@@ -2209,15 +2217,19 @@ pm_status plain_residual_norm(pm_mg* mg, const float* phi, double* out, hipStrea
 pm_status mixed_residual(pm_mg* mg, const float* phi, hipStream_t s, bool split = false,
                          bool defer = false) {
   const Level& L = mg->lv[0];
-  // 8 nodes per thread on split grids with n % 8 == 0 and 16-byte aligned phi and rho
-  const bool quad = split && mg->quad_blocks && (reinterpret_cast<uintptr_t>(phi) & 15u) == 0 &&
+  // 8 nodes per thread on grids with n % 8 == 0 and 16-byte aligned phi and rho
+  const bool quad = mg->quad_blocks && (reinterpret_cast<uintptr_t>(phi) & 15u) == 0 &&
                     (reinterpret_cast<uintptr_t>(mg->cur_rho) & 15u) == 0;
   const unsigned b = quad ? mg->res_blocks : pm::red_blocks(L.nodes());
   double* partials = quad ? (defer ? mg->partials_r : mg->partials_q) : mg->partials;
   {
     PM_TIMED("mg.residual64", kRes64Bytes * L.nodes(), s);
-    if (quad)
-      residual64_s4_kernel<<<b, pm::kBlock, 0, s>>>(phi, mg->cur_rho, mg->factor, L.n, mg->hn,
+    if (quad && !split)
+      residual64_s4_kernel<false><<<b, pm::kBlock, 0, s>>>(phi, mg->cur_rho, mg->factor, L.n,
+                                                           mg->hn, 1.0 / (L.h * L.h), mg->r32,
+                                                           partials);
+    else if (quad)
+      residual64_s4_kernel<true><<<b, pm::kBlock, 0, s>>>(phi, mg->cur_rho, mg->factor, L.n, mg->hn,
                                                      1.0 / (L.h * L.h),
                                                      mg->r32s, partials);
     else if (split)
@@ -2353,8 +2365,8 @@ pm_status mixed_correct(pm_mg* mg, float* phi, double v[4], hipStream_t s,
 }
 
 // Moments, f = 4*pi*G*rho, the initial guess (zero unless warm) with multipole faces, and
-// ||f|| (into red[3]). Enqueued only. f is stored in f0 for the PLAIN cycle and the
-// network's input (store_f); the MIXED defect scales rho itself with the same float product.
+// ||f|| (into red[3]). Enqueued only. f is stored in f0 for the PLAIN cycle (store_f); the
+// MIXED defect and the network's input scale rho themselves with the same float product.
 pm_status solve_setup(pm_mg* mg, const float* rho, float* phi, bool warm, hipStream_t s,
                       bool store_f) {
   Level& L0 = mg->lv[0];
@@ -2385,11 +2397,13 @@ pm_status solve_setup(pm_mg* mg, const float* rho, float* phi, bool warm, hipStr
 }
 
 // The V-cycle loop of a solve whose setup has run (PLAIN: reference stop rule; MIXED:
-// defect correction with the error-estimate stop). Fills stats. residual_ready: MIXED only,
-// r32 already holds the defect of phi and red[2] its squared norm. carry: MIXED only, the
+// defect correction with the error-estimate stop). Fills stats. ready: MIXED only, r32
+// (kDefectNatural) or r32s (kDefectSplit) already holds the defect of phi and red[2] its
+// squared norm. carry: MIXED only, the
 // solve starts from mg->guess and its corrections carry the next guess (kCycleCarry*).
+enum { kDefectNone = 0, kDefectNatural = 1, kDefectSplit = 2 };
 pm_status solve_iterate(pm_mg* mg, float* phi, pm_mg_stats* stats, hipStream_t s,
-                        bool residual_ready = false, bool carry = false) {
+                        int ready = kDefectNone, bool carry = false) {
   Level& L0 = mg->lv[0];
   const bool mixed = mg->d.mode == PM_MG_MIXED;
   pm_status st;
@@ -2439,12 +2453,16 @@ pm_status solve_iterate(pm_mg* mg, float* phi, pm_mg_stats* stats, hipStream_t s
     auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const bool defer = carry && split && mg->quad_blocks && aligned(phi) && aligned(mg->guess) &&
                        aligned(mg->cur_rho);
-    if (!residual_ready) {
+    if (ready == kDefectNone) {
       if ((st = mixed_residual(mg, carry ? mg->guess : phi, s, split, defer))) return st;
-    } else if (split) {
+    } else if (split && ready == kDefectNatural) {
       PM_TIMED("mg.to_split", 8.0 * L0.nodes(), s);
-      to_split_kernel<<<pm::blocks_for(L0.nodes()), pm::kBlock, 0, s>>>(mg->r32, mg->r32s,
-                                                                        L0.n, mg->hn);
+      if (L0.n % 8 == 0)
+        to_split4_kernel<<<pm::blocks_for(L0.nodes() / 8), pm::kBlock, 0, s>>>(mg->r32, mg->r32s,
+                                                                               L0.n, mg->hn);
+      else
+        to_split_kernel<<<pm::blocks_for(L0.nodes()), pm::kBlock, 0, s>>>(mg->r32, mg->r32s, L0.n,
+                                                                          mg->hn);
       PM_CHECK_LAUNCH("to_split_kernel");
     }
     double prev_e = -1.0;
@@ -2748,14 +2766,13 @@ pm_status pm_mg_solve_warm(pm_mg* mg, const float* rho, float* phi, pm_mg_warm* 
     mg->guess_valid = false;
     if ((st = solve_setup(mg, rho, mg->guess, true, s, false))) return st;  // faces into it
     w->extrapolated = have ? 1 : 0;
-    if ((st = solve_iterate(mg, phi, stats, s, false, true))) return st;
+    if ((st = solve_iterate(mg, phi, stats, s, kDefectNone, true))) return st;
     mg->guess_valid = mg->d.n_cycles > 0;
     mg->guess_phi = phi;
     return PM_OK;
   }
   mg->guess_valid = false;
-  if ((st = solve_setup(mg, rho, phi, true, s, mg->d.mode == PM_MG_PLAIN || want_net_grid)))
-    return st;
+  if ((st = solve_setup(mg, rho, phi, true, s, mg->d.mode == PM_MG_PLAIN))) return st;
   const bool extrap = w->mode != PM_WARM_PREVIOUS && mg->hist_valid;
   if (!extrap) {
     // first solve of a sequence (or PREVIOUS mode): phi itself is the guess; remember it
@@ -2764,12 +2781,14 @@ pm_status pm_mg_solve_warm(pm_mg* mg, const float* rho, float* phi, pm_mg_warm* 
     return solve_iterate(mg, phi, stats, s);
   }
   w->extrapolated = 1;
-  if ((st = pm::warm::extrapolate(phi, mg->hist, (learned || w->pair_target) ? mg->cand : nullptr,
+  // the MIXED loop can start from the defect computed below (of phi, corrected or not)
+  int ready = want_net_grid && mg->d.mode == PM_MG_MIXED ? kDefectNatural : kDefectNone;
+  if ((st = pm::warm::extrapolate(phi, mg->hist, w->pair_target ? mg->cand : nullptr,
                                   n, s)))
     return st;
   if (want_net_grid) {
     if ((st = mixed_residual(mg, phi, s))) return st;  // r32, ||r||^2 -> red[2]
-    if ((st = pm::warm::make_input(mg->r32, phi, mg->hist, mg->f0, n, w->pool, L0.h, mg->pooled,
+    if ((st = pm::warm::make_input(mg->r32, phi, mg->hist, rho, mg->factor, n, w->pool, L0.h, mg->pooled,
                                    mg->net_in, mg->partials, mg->red + 4, mg->scales, s)))
       return st;
     if (w->pair_input) {
@@ -2781,10 +2800,12 @@ pm_status pm_mg_solve_warm(pm_mg* mg, const float* rho, float* phi, pm_mg_warm* 
   }
   if (learned) {
     if ((st = pm_wsnet_forward(w->net, mg->net_in, mg->net_out, s))) return st;
-    if ((st = pm::warm::apply(mg->net_out, n, w->pool, mg->scales, mg->e0, s))) return st;
-    // the judge also writes the corrected guess's residual into the level-0 scratch
+    // the judge also writes the corrected guess's residual: split where the cycles take it
+    // split, else into the level-0 scratch
     Level& lv0 = mg->lv[0];
-    if ((st = pm::warm::guard(mg->r32, mg->e0, n, w->pool, L0.h, lv0.res, mg->partials,
+    const bool split = mg->d.mode == PM_MG_MIXED && mg->split_active();
+    if ((st = pm::warm::guard(mg->r32, mg->net_out, n, w->pool, L0.h, mg->scales, mg->e0,
+                              split ? mg->r32s : lv0.res, split ? mg->hn : 0, mg->partials,
                               mg->red + 8, s)))
       return st;
     double v[11];  // red[8], red[9]: pooled residual before / after; red[10]: ||r after||^2
@@ -2792,21 +2813,17 @@ pm_status pm_mg_solve_warm(pm_mg* mg, const float* rho, float* phi, pm_mg_warm* 
     w->resid_before = std::sqrt(v[8]);
     w->resid_after = std::sqrt(v[9]);
     if (std::isfinite(w->resid_after) && w->resid_after < w->fallback_ratio * w->resid_before) {
-      const unsigned b = pm::red_blocks(nodes);
-      {
-        PM_TIMED("mg.update", kUpdBytes * nodes, s);
-        update_kernel<kCarryNone><<<b, pm::kBlock, 0, s>>>(phi, mg->e0, nullptr, nodes,
-                                                           mg->partials);
-        PM_CHECK_LAUNCH("update_kernel");
+      if ((st = pm::warm::correct(phi, mg->net_out, n, w->pool, mg->scales, mg->e0, s))) return st;
+      if (split) {
+        ready = kDefectSplit;
+      } else {
+        std::swap(mg->r32, lv0.res);  // the defect of the corrected phi
       }
-      std::swap(mg->r32, lv0.res);  // the defect of the corrected phi
       PM_TRY_HIP(hipMemcpyAsync(mg->red + 2, mg->red + 10, sizeof(double),
                                 hipMemcpyDeviceToDevice, s));
       w->used_net = 1;
     }
   }
-  // the MIXED loop can start from the defect computed above (of phi, corrected or not)
-  const bool ready = want_net_grid && mg->d.mode == PM_MG_MIXED;
   if ((st = solve_iterate(mg, phi, stats, s, ready))) return st;
   if (w->pair_target)
     return pm::warm::target(phi, mg->cand, n, w->pool, mg->scales, w->pair_target, s);

@@ -282,3 +282,72 @@ def test_carried_guess_equals_extrapolation_pass(device, seq_b):
                 assert carried.last_warm["extrapolated"] and explicit.last_warm["extrapolated"]
                 assert not explicit.last_warm["used_net"]
             assert torch.equal(pa, pb), (split, t)
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("n,pool", [(64, 1), (48, 2), (64, 2), (64, 4), (96, 4), (72, 1),
+                                    (64, 8), (192, 8), (128, 16)])
+def test_network_correction_and_its_judge(device, n, pool, split):
+    """The correction added to the guess and the judge's pooled residuals, recomputed in
+    float64 from the network's own output, for every pool factor that has its own path, one
+    wave's worth of nodes along k and less or more.
+
+    Bounds: e takes about ten float32 roundings of values up to max|e| and is added to phi once:
+    2e-6 * max|e| + 2^-23 * max|phi|. The residual after it feels e's error through 12 / h^2:
+    about 2.4e-5 * pool^2 * max|out| of the residual's RMS, a few 1e-4 at pool 16: 1e-3."""
+    announce(f"network correction n={n} pool={pool} split={split}")
+    from galaxy_collision_amd import _native as nat
+    from galaxy_collision_amd.solver.multigrid import MixedPrecisionMultigridSolver
+    from galaxy_collision_amd.warmstart import WarmStartNet
+
+    R, h = n // pool, 20.0 / n
+    net = WarmStartNet(R, seed=3)
+    s = MixedPrecisionMultigridSolver(n, dx=h, grav_constant=1.0, warm="learned", net=net,
+                                      pool=pool, fallback_ratio=1e30, n_cycles=0,
+                                      split_fine=split)
+    g = torch.Generator().manual_seed(n + pool)
+    rho = torch.rand((n,) * 3, generator=g).to(device)
+    phi = torch.rand((n,) * 3, generator=g).to(device)
+    s.solve_warm(rho, phi, nat.PM_WARM_LEARNED)
+    hist = phi.clone()
+    phi += 0.1 * torch.rand((n,) * 3, generator=g).to(device)
+    before = phi.clone()
+    x = torch.empty((R ** 3, 8), dtype=torch.bfloat16, device=device)
+    rec = s.solve_warm(rho, phi, nat.PM_WARM_LEARNED, x)
+    assert rec["extrapolated"] and rec["used_net"]
+    out = net.forward(x.view(R, R, R, 8)).double().reshape(R, R, R)
+    # the guess: faces of this solve, 2 phi - hist inside
+    guess = phi.double()
+    inner = (slice(1, -1),) * 3
+    guess[inner] = (2.0 * before[inner] - hist[inner]).double()
+
+    def lap(u):
+        return (u[2:, 1:-1, 1:-1] + u[:-2, 1:-1, 1:-1] + u[1:-1, 2:, 1:-1] + u[1:-1, :-2, 1:-1] +
+                u[1:-1, 1:-1, 2:] + u[1:-1, 1:-1, :-2] - 6.0 * u[inner]) / (h * h)
+
+    def pooled(v):
+        f = torch.zeros((n,) * 3, dtype=torch.float64, device=device)
+        f[inner] = v
+        return F.avg_pool3d(f[None, None], pool)
+
+    r = (F32(4.0 * math.pi) * rho).double()[inner] - lap(guess)
+    rms = float(pooled(r).pow(2).mean().sqrt())
+    u = (2 * torch.arange(n, device=device) - (pool - 1)).double() / (2 * pool)
+    lo = u.floor()
+    w = u - lo
+    lo = lo.long()
+    i0, i1 = lo.clamp(0, R - 1), (lo + 1).clamp(0, R - 1)
+    e = out
+    for axis in (2, 1, 0):
+        shape = [1, 1, 1]
+        shape[axis] = n
+        wa = w.view(shape)
+        e = e.index_select(axis, i0) * (1 - wa) + e.index_select(axis, i1) * wa
+    full = torch.zeros_like(guess)
+    full[inner] = rms * (pool * h) ** 2 * e[inner]
+    got = phi.double() - guess
+    tol = 2e-6 * float(full.abs().max()) + 2.0 ** -23 * float(phi.abs().max())
+    assert float((got - full).abs().max()) <= tol
+    assert rec["resid_before"] == pytest.approx(float(pooled(r).pow(2).sum().sqrt()), rel=1e-3)
+    after = pooled(r - lap(full)).pow(2).sum().sqrt()
+    assert rec["resid_after"] == pytest.approx(float(after), rel=1e-3)
