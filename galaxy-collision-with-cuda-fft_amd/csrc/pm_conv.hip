@@ -416,9 +416,17 @@ struct ConvWgradArgs {
 // one voxel range; wave w owns columns 16w..16w+15. The first column group's wave 0 also
 // multiplies dz with ones: the bias gradient's sums ride on operands it has loaded anyway
 // (a pass of their own took 31-118 us a layer at 64^3-16^3, as long as this kernel).
-template <int NR>
+//
+// A stage of V voxels is loaded a stage ahead into registers and transposed into LDS as pairs of
+// voxels (one 32-bit write per two); both operands then come from LDS for V/32 products. Staging
+// 32 voxels at a time with their loads waited for in place, and coordinates by division, took 60
+// us a call over the layers of 16 channels at 64^3-8^3 (now 38), 22 at 32 channels (18), 16 at
+// 64 (14). Above 64 rows the LDS tile and the few voxels of those layers want V = 64.
+template <int NR, int V>
 __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
-  constexpr int kLd = 40;  // 32 voxels + 8 pad (80-byte rows keep 16-byte alignment)
+  constexpr int kLd = V + 8;       // row stride: keeps 16-byte alignment
+  constexpr int kXP = V / 64;      // voxel pairs of x per thread and stage
+  constexpr int kDP = NR * V >= 256 ? NR * V / 256 : 1;  // pair loads of dz per thread, at most
   __shared__ __align__(16) uint16_t sdz[NR * 16][kLd];
   __shared__ __align__(16) uint16_t sx[64][kLd];
   const int tid = threadIdx.x;
@@ -429,7 +437,7 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
 
   for (int p = tid; p < NR * 16 * kLd; p += 256) (&sdz[0][0])[p] = 0;  // rows >= dz_c stay 0
 
-  const int cg = tid >> 5, vs = tid & 31;  // x staging: column group (8 columns), voxel slot
+  const int cg = tid >> 5, vs = tid & 31;  // x staging: column group (8 columns), pair slot
   const int kq = k0 + 8 * cg;
   const bool kvalid = kq < a.kreal;
   int ci = 0, dz = 0, dy = 0, dx = 0;
@@ -440,7 +448,9 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
     dy = (tap / 3) % 3 - 1;
     dx = tap % 3 - 1;
   }
-  const int c8n = a.dz_c >> 3;
+  const int c8s = __builtin_ctz(static_cast<unsigned>(a.dz_c)) - 3;  // dz_c / 8 = 1 << c8s
+  const bool pow2 = (a.r & (a.r - 1)) == 0;
+  const int rs = __builtin_ctz(static_cast<unsigned>(a.r));
   f32x4_t acc[NR];
 #pragma unroll
   for (int rb = 0; rb < NR; ++rb) acc[rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -452,40 +462,72 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
 
   const int vbeg = split * a.chunks_per_split * 32;
   const int vend = min(a.nvox, vbeg + a.chunks_per_split * 32);
-  for (int vc = vbeg; vc < vend; vc += 32) {
-    __syncthreads();  // previous chunk's MFMA reads are done (and the zero fill above)
-    for (int p = tid; p < 32 * c8n; p += 256) {
-      const int v = p / c8n, c8 = p - v * c8n;
-      u32x4_t val{0u, 0u, 0u, 0u};
-      if (vc + v < a.nvox) val = load16(a.dz + static_cast<int64_t>(vc + v) * a.dz_c + 8 * c8);
+  u32x4_t xr[kXP][2], dr[kDP][2];
+  auto load_stage = [&](int vc) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        sdz[8 * c8 + 2 * q][v] = static_cast<uint16_t>(val[q] & 0xffffu);
-        sdz[8 * c8 + 2 * q + 1][v] = static_cast<uint16_t>(val[q] >> 16);
-      }
-    }
-    {
-      u32x4_t val{0u, 0u, 0u, 0u};
-      const int v = vc + vs;
-      if (kvalid && v < a.nvox) {
-        const int x = v % a.r, y = (v / a.r) % a.r, z = v / (a.r * a.r);
-        const uint16_t* p =
-            conv_src(a.xa, a.xb, a.ca, a.cb, a.r, a.ra, a.up, z + dz, y + dy, x + dx, ci);
-        if (p) val = load16(p);
+    for (int m = 0; m < kXP; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int v = vc + 64 * m + 2 * vs + h;
+        xr[m][h] = u32x4_t{0u, 0u, 0u, 0u};
+        if (kvalid && v < vend) {
+          int x, y, z;
+          if (pow2) {
+            x = v & (a.r - 1);
+            y = (v >> rs) & (a.r - 1);
+            z = v >> (2 * rs);
+          } else {
+            x = v % a.r;
+            y = (v / a.r) % a.r;
+            z = v / (a.r * a.r);
+          }
+          const uint16_t* p =
+              conv_src(a.xa, a.xb, a.ca, a.cb, a.r, a.ra, a.up, z + dz, y + dy, x + dx, ci);
+          if (p) xr[m][h] = load16(p);
+        }
       }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        sx[8 * cg + 2 * q][vs] = static_cast<uint16_t>(val[q] & 0xffffu);
-        sx[8 * cg + 2 * q + 1][vs] = static_cast<uint16_t>(val[q] >> 16);
+    for (int m = 0; m < kDP; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int p = tid + 256 * m, vp = p >> c8s, c8 = p & ((1 << c8s) - 1);
+        const int v = vc + 2 * vp + h;
+        dr[m][h] = u32x4_t{0u, 0u, 0u, 0u};
+        if (vp < V / 2 && v < vend)
+          dr[m][h] = load16(a.dz + static_cast<int64_t>(v) * a.dz_c + 8 * c8);
       }
+  };
+  // channels 8q..8q+7 of a voxel pair into 8 rows, one 32-bit write each
+  auto put = [&](uint16_t* dst, const u32x4_t& lo, const u32x4_t& hi) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      *reinterpret_cast<uint32_t*>(dst + (2 * q) * kLd) = (lo[q] & 0xffffu) | (hi[q] << 16);
+      *reinterpret_cast<uint32_t*>(dst + (2 * q + 1) * kLd) = (lo[q] >> 16) | (hi[q] & 0xffff0000u);
     }
+  };
+  if (vbeg < vend) load_stage(vbeg);
+  for (int vc = vbeg; vc < vend; vc += V) {
+    __syncthreads();  // the previous stage's MFMA reads are done (and the zero fill above)
+#pragma unroll
+    for (int m = 0; m < kDP; ++m) {
+      const int p = tid + 256 * m, vp = p >> c8s, c8 = p & ((1 << c8s) - 1);
+      if (vp < V / 2) put(&sdz[8 * c8][2 * vp], dr[m][0], dr[m][1]);
+    }
+#pragma unroll
+    for (int m = 0; m < kXP; ++m) put(&sx[8 * cg][64 * m + 2 * vs], xr[m][0], xr[m][1]);
     __syncthreads();
-    const u32x4_t bq = *reinterpret_cast<const u32x4_t*>(&sx[16 * wave + row][8 * grp]);
+    if (vc + V < vend) load_stage(vc + V);
 #pragma unroll
-    for (int rb = 0; rb < NR; ++rb) {
-      const u32x4_t aq = *reinterpret_cast<const u32x4_t*>(&sdz[16 * rb + row][8 * grp]);
-      acc[rb] = mfma_bf16(aq, bq, acc[rb]);
-      if (sums) accb[rb] = mfma_bf16(aq, ones, accb[rb]);
+    for (int q = 0; q < V / 32; ++q) {
+      if (vc + 32 * q >= vend) break;
+      const u32x4_t bq = *reinterpret_cast<const u32x4_t*>(&sx[16 * wave + row][32 * q + 8 * grp]);
+#pragma unroll
+      for (int rb = 0; rb < NR; ++rb) {
+        const u32x4_t aq =
+            *reinterpret_cast<const u32x4_t*>(&sdz[16 * rb + row][32 * q + 8 * grp]);
+        acc[rb] = mfma_bf16(aq, bq, acc[rb]);
+        if (sums) accb[rb] = mfma_bf16(aq, ones, accb[rb]);
+      }
     }
   }
   if (sums && row == 0) {  // every column holds the same sums
@@ -510,7 +552,7 @@ __global__ void __launch_bounds__(256) conv_wgrad_kernel(ConvWgradArgs a) {
 // last grid row: 64 channels of the bias); the kFoldWaves waves take every kFoldWaves-th split,
 // a few loads in flight at once, and their sums are added in wave order (deterministic). One
 // thread that walked all splits of an output kept a load at a time in flight: 80 us for the
-// 283 splits of a 64^3 layer of 16 channels, 157 us for 512.
+// 283 splits that a 64^3 layer of 16 channels had, 157 us for 512.
 constexpr int kFoldWaves = 16;
 __global__ void __launch_bounds__(64 * kFoldWaves) wgrad_fold_kernel(
     const float* __restrict__ partial, const float* __restrict__ partial_b, int splits, int cout,
@@ -826,12 +868,15 @@ int64_t wgrad_partial_floats(int cin, int cout, int r) {
   return static_cast<int64_t>(splits) * rows * (kcols + 1);  // and the channel sums
 }
 
+// About 1024 workgroups, 4 per CU: with 2048 the stages are too few to hide their loads and the
+// fold reads twice the partial sums (weight gradients of a 4-pair batch 1.95 ms against 1.88),
+// with 512 too few loads are in flight (2.29 ms).
 void wgrad_plan(int cin, int cout, int r, int* splits, int* chunks_per_split) {
   (void)cout;
   const int64_t nvox = static_cast<int64_t>(r) * r * r;
   const int64_t nchunks = (nvox + 31) / 32;
   const int kgroups = (kpad(cin) + 63) / 64;
-  int64_t want = std::max<int64_t>(1, 2048 / kgroups);
+  int64_t want = std::max<int64_t>(1, 1024 / kgroups);
   want = std::min<int64_t>(want, nchunks);
   const int64_t per = (nchunks + want - 1) / want;
   *chunks_per_split = static_cast<int>(per);
@@ -878,10 +923,10 @@ pm_status wgrad(const uint16_t* xa, int ca, const uint16_t* xb, int cb, int r, i
     const double flops = 2.0 * 27.0 * cin * cout * static_cast<double>(a.nvox);
     PM_TIMED(timer, flops, s);
     switch (nr) {
-      case 1: conv_wgrad_kernel<1><<<grid, 256, 0, s>>>(a); break;
-      case 2: conv_wgrad_kernel<2><<<grid, 256, 0, s>>>(a); break;
-      case 4: conv_wgrad_kernel<4><<<grid, 256, 0, s>>>(a); break;
-      default: conv_wgrad_kernel<8><<<grid, 256, 0, s>>>(a); break;
+      case 1: conv_wgrad_kernel<1, 128><<<grid, 256, 0, s>>>(a); break;
+      case 2: conv_wgrad_kernel<2, 128><<<grid, 256, 0, s>>>(a); break;
+      case 4: conv_wgrad_kernel<4, 64><<<grid, 256, 0, s>>>(a); break;
+      default: conv_wgrad_kernel<8, 64><<<grid, 256, 0, s>>>(a); break;
     }
     PM_CHECK_LAUNCH("conv_wgrad_kernel");
   }

@@ -276,3 +276,34 @@ def test_conv_argument_checks(device):
 def test_conv_tile_edges_match_float64(device, r, ca, cb, up, cout, act):
     """Tile borders, halves of a chunk in two taps, channel slices and the fallback."""
     test_conv_forward_matches_float64(device, r, ca, cb, up, cout, act, False)
+
+
+@pytest.mark.parametrize("r,cin,cout", [(24, 16, 16), (40, 8, 1), (32, 16, 29), (24, 40, 32),
+                                        (24, 16, 64), (12, 64, 60), (24, 8, 128), (9, 24, 121)])
+def test_weight_gradient_stages_match_float64(device, r, cin, cout):
+    """Several stages per workgroup with a ragged last one, edges that are no power of two, every
+    row count (16 to 128), columns that end inside a group. Float32 sums of up to 64,000 products
+    of bf16 values, split and then folded: relative error about 1e-6, bound 1e-5."""
+    announce(f"conv wgrad stages r={r} cin={cin} cout={cout}")
+    nat = _nat()
+    g = torch.Generator().manual_seed(11 + r + cin + cout)
+    x = bf16_rand((r ** 3, cin), g)
+    dz = torch.zeros(r ** 3, store(cout), dtype=torch.bfloat16)
+    dz[:, :cout] = bf16_rand((r ** 3, cout), g)
+    w = torch.zeros(cout, cin, 3, 3, 3, dtype=torch.float64, requires_grad=True)
+    b = torch.zeros(cout, dtype=torch.float64, requires_grad=True)
+    y = F.conv3d(concat_input(x, cin, None, 0, r, 0), w, b, padding=1)
+    (y * to_ncdhw(dz[:, :cout].contiguous(), r)).sum().backward()
+    nfl = ctypes.c_int64()
+    nat.call("pm_conv3d_wgrad_partial_size", cin, cout, r, ctypes.byref(nfl))
+    part = torch.empty(nfl.value, dtype=torch.float32, device=device)
+    dw = torch.empty(cout * cin * 27, dtype=torch.float32, device=device)
+    db = torch.empty(cout, dtype=torch.float32, device=device)
+    x_d, dz_d = x.to(device), dz.reshape(-1).to(device)
+    nat.call("pm_conv3d_bwd_weight_bf16", nat.ptr(x_d, torch.bfloat16), cin, None, 0, r, 0,
+             nat.ptr(dz_d, torch.bfloat16), cout, nat.ptr(dw), nat.ptr(db), 0, nat.ptr(part),
+             nfl.value, nat.stream())
+    torch.cuda.synchronize()
+    assert rel_l2(dw.cpu().numpy().reshape(cout, cin, 27),
+                  w.grad.numpy().reshape(cout, cin, 27)) < 1e-5
+    np.testing.assert_allclose(db.cpu().numpy(), b.grad.numpy(), rtol=1e-5, atol=1e-4)
