@@ -307,3 +307,40 @@ def test_weight_gradient_stages_match_float64(device, r, cin, cout):
     assert rel_l2(dw.cpu().numpy().reshape(cout, cin, 27),
                   w.grad.numpy().reshape(cout, cin, 27)) < 1e-5
     np.testing.assert_allclose(db.cpu().numpy(), b.grad.numpy(), rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("r,gc,dz_c,stride,shift", [(6, 16, 16, 16, 0), (10, 8, 16, 12, 0),
+                                                    (8, 24, 32, 24, 0), (8, 24, 32, 26, 0),
+                                                    (6, 16, 16, 16, 1), (6, 1, 8, 1, 0),
+                                                    (4, 128, 128, 192, 0)])
+@pytest.mark.parametrize("use", ["g1", "g2", "g1 y", "g1 g2 y"])
+def test_act_bwd_widths(device, r, gc, dz_c, stride, shift, use):
+    """8 channels a thread where channels, strides and alignment allow it, one where they do not
+    (gc = 1, stride 26, arrays shifted by one element): exactly the float32 expression."""
+    announce(f"act_bwd r={r} gc={gc} dz_c={dz_c} stride={stride} shift={shift} use={use}")
+    nat = _nat()
+    g = torch.Generator().manual_seed(r + gc)
+    g1, g2 = torch.randn(r ** 3, stride, generator=g), torch.randn((r // 2) ** 3, gc, generator=g)
+    act = bf16_rand((r ** 3, gc), g)
+
+    def dev(t):
+        buf = torch.zeros(t.numel() + shift, dtype=t.dtype, device=device)
+        buf[shift:] = t.reshape(-1).to(device)
+        return buf[shift:]
+
+    g1_d, g2_d, act_d = dev(g1), dev(g2), dev(act)
+    dz = torch.full((r ** 3 * dz_c,), 7.0, dtype=torch.bfloat16, device=device)
+    nat.call("pm_act_bwd_bf16", nat.ptr(g1_d) if "g1" in use else None, stride,
+             nat.ptr(g2_d) if "g2" in use else None,
+             nat.ptr(act_d, torch.bfloat16) if "y" in use else None, 0.1, r, gc, dz_c,
+             nat.ptr(dz, torch.bfloat16), nat.stream())
+    want = g1[:, :gc].clone() if "g1" in use else torch.zeros(r ** 3, gc)
+    if "g2" in use:
+        up = to_cl(to_ncdhw(g2, r // 2).repeat_interleave(2, 2).repeat_interleave(2, 3)
+                   .repeat_interleave(2, 4)).float()
+        want = want + up * 0.125
+    if "y" in use:
+        want = want * torch.where(act.float() > 0, 1.0, 0.1)
+    got = dz.cpu().view(-1, dz_c)
+    assert torch.equal(got[:, :gc], want.to(torch.bfloat16))
+    assert not got[:, gc:].float().any()
