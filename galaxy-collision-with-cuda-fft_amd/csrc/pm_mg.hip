@@ -2510,7 +2510,8 @@ pm_status solve_iterate(pm_mg* mg, float* phi, pm_mg_stats* stats, hipStream_t s
 // PLAIN grids from this size on (multiples of 8) run their cycles with the finest level in split
 // layout: a colour pass reads and writes half of what the natural one does (256^3 34 -> 18 us,
 // 128^3 7.5 -> 4.1; residual 36 -> 31, prolongation 52 -> 21), and the solve pays three copies
-// for it (21 us at 128^3). A cold 256^3 solve of 20 cycles 11.8 -> 8.5 ms; one warm cycle at
+// for it (21 us at 128^3). A cold 256^3 solve of 20 cycles 11.8 -> 8.5 ms by the layout alone (7.4
+// with the residual and restriction fused and the coarse levels split too); one warm cycle at
 // 128^3 gains 9 us of a 400 us step. At 64^3 a pass is all latency (3.5 us either way).
 constexpr int kPlainSplitMin = 96;
 

@@ -21,7 +21,7 @@
 // up to 17^3). Measured per leg on the MI355X, us, against the per-pass kernels it replaces:
 // 33^3 V(1,1) 4.8 down, 5.8 up (9.5, 7.5), V(2,2) 8.4, 9.8 (13, 12); 65^3 V(1,1) 6.2, 6.9
 // (9.9, 8.3), V(2,2) 11.7, 13.3 (14.7, 13.0). At 129^3 V(2,2) the leg takes 60 and 73 us against 39 and 40, and 16^3
-// blocks 41 and 41: levels above kLegMax keep the passes. 4^3 blocks measured 4.0 and 4.2 us at
+// blocks 41 and 41: levels above kLegMax keep a launch per pass. 4^3 blocks measured 4.0 and 4.2 us at
 // 33^3 V(1,1) but 8.4 and 9.1 at V(2,2) and lost from 41^3 up.
 #pragma once
 
