@@ -48,18 +48,25 @@ struct BigCell {
 // ---------------------------------------------------------------------------------------
 //
 // REC: also the particle's record for the piece pass, its offsets in its cell and its mass per
-// cell volume. The piece pass reads particles in key order; from the four arrays that is four
-// scattered lines for a particle whose neighbours in memory are elsewhere, from the records one
-// (3M particles in random order on 192^3: a deposit 330 -> 230 us).
+// cell volume, unless *ordered says that the particles lie in cell order (null: always). The
+// piece pass reads particles in key order; from the four arrays that is four scattered lines for
+// a particle whose neighbours in memory are elsewhere, from the records one (a deposit of 3M
+// particles in random order on 192^3 357 us without records, 230 with; 10M on 256^3 1087, 607).
+// Particles in cell order share their lines, and the 20 bytes more that the key pass moves for
+// each cost more than the piece pass saves (10M: key pass 37 us without, 76 with, piece pass 66
+// and 60, deposit 345 and 380).
 template <bool REC>
 __global__ void __launch_bounds__(256) key_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const float* __restrict__ mass, float inv_vol, int64_t np, int n, float dx, uint32_t sentinel,
-    uint32_t* __restrict__ keys, uint32_t* __restrict__ keys_out, float4* __restrict__ rec) {
+    uint32_t* __restrict__ keys, uint32_t* __restrict__ keys_out, float4* __restrict__ rec,
+    const int* __restrict__ ordered) {
   const int64_t p = pm::xcd_block() * blockDim.x + threadIdx.x;
   if (p >= np) return;
   // all loads first (the && below would otherwise order them)
-  const float x = px[p], y = py[p], z = pz[p], w = REC ? mass[p] : 0.0f;
+  const float x = px[p], y = py[p], z = pz[p];
+  const bool keep = REC && !(ordered && *ordered);
+  const float w = keep ? mass[p] : 0.0f;
   int ix = 0, iy = 0, iz = 0;
   float fx = 0.0f, fy = 0.0f, fz = 0.0f;
   const bool in = pm::cic_axis(x, dx, n, ix, fx) && pm::cic_axis(y, dx, n, iy, fy) &&
@@ -67,9 +74,39 @@ __global__ void __launch_bounds__(256) key_kernel(
   const uint32_t key = in ? pm::cell_key(ix, iy, iz, n) : sentinel;
   keys[p] = key;
   if (keys_out) keys_out[p] = key;
-  if (REC) rec[p] = make_float4(fx, fy, fz, w * inv_vol);
+  if (keep) rec[p] = make_float4(fx, fy, fz, w * inv_vol);
 }
 
+// Whether the particles lie in cell order, for one wave: at least 7 of 8 sampled neighbours in
+// memory (64 pairs spread over the arrays, np >= 2) have ascending keys. Random order gives half
+// of them. The records' line lies near a displacement of 0.2 cells from cell order (10M on
+// 256^3, deposit in us with / without: in order 380 / 345, displaced by 0.1 cells rms 403 / 394,
+// by 0.25 431 / 435, by 0.5 453 / 481, by 1 484 / 604).
+struct OrderSample {
+  const float* px;
+  const float* py;
+  const float* pz;
+  int64_t np;
+  float dx;
+  uint32_t sentinel;
+  int* ordered;  // null: not asked for
+};
+
+__device__ __forceinline__ void sample_order(const OrderSample& s, int n) {
+  const int64_t p = (s.np - 1) * static_cast<int64_t>(threadIdx.x & 63u) / 64;
+  uint32_t key[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float x = s.px[p + h], y = s.py[p + h], z = s.pz[p + h];
+    int ix = 0, iy = 0, iz = 0;
+    float f;
+    const bool in = pm::cic_axis(x, s.dx, n, ix, f) && pm::cic_axis(y, s.dx, n, iy, f) &&
+                    pm::cic_axis(z, s.dx, n, iz, f);
+    key[h] = in ? pm::cell_key(ix, iy, iz, n) : s.sentinel;
+  }
+  const int up = __popcll(__ballot(key[0] <= key[1]));
+  if ((threadIdx.x & 63u) == 0) *s.ordered = up >= 56 ? 1 : 0;
+}
 
 // ---------------------------------------------------------------------------------------
 // 2. stable LSD radix sort (reduce-then-scan; no inter-workgroup waiting)
@@ -375,7 +412,8 @@ template <bool REC>
 __global__ void __launch_bounds__(256) piece_kernel(
     const uint32_t* __restrict__ skey, const int32_t* __restrict__ sidx,
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
-    const float* __restrict__ mass, const float4* __restrict__ rec, float dx, float inv_vol, int64_t np, uint32_t sentinel,
+    const float* __restrict__ mass, const float4* __restrict__ rec,
+    const int* __restrict__ ordered, float dx, float inv_vol, int64_t np, uint32_t sentinel,
     int64_t chunks, float* __restrict__ sums, int32_t* __restrict__ map,
     float* __restrict__ head, float* __restrict__ tail, int64_t* __restrict__ tail_slot,
     uint8_t* __restrict__ head_end, int n, uint8_t* __restrict__ bricks, pm::FastDiv m1) {
@@ -398,38 +436,32 @@ __global__ void __launch_bounds__(256) piece_kernel(
     key[r] = g < np ? skey[g] : 0xFFFFFFFFu;
     q[r] = g < np ? sidx[g] : 0;
   }
-  float x[kPer], y[kPer], z[kPer], w[kPer];
+  // one branch around all loads of either kind (one per position kept the second position's
+  // loads waiting for the first's: 114 -> 154 us for 10M particles displaced by a cell)
+  float4 v[kPer];
+  if (REC && !(ordered && *ordered)) {
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    if (REC) {
-      const float4 v = rec[q[r]];
-      x[r] = v.x;
-      y[r] = v.y;
-      z[r] = v.z;
-      w[r] = v.w;
-      continue;
+    for (int r = 0; r < kPer; ++r) v[r] = rec[q[r]];
+  } else {
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) v[r] = make_float4(px[q[r]], py[q[r]], pz[q[r]], mass[q[r]]);
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      // the particle's offsets in its cell, recomputed from its coordinates exactly as its
+      // key was (a live key means all three axes are in range; others are not used)
+      int ix, iy, iz;
+      float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+      (void)pm::cic_axis(v[r].x, dx, n, ix, fx);
+      (void)pm::cic_axis(v[r].y, dx, n, iy, fy);
+      (void)pm::cic_axis(v[r].z, dx, n, iz, fz);
+      v[r] = make_float4(fx, fy, fz, v[r].w * inv_vol);
     }
-    x[r] = px[q[r]];
-    y[r] = py[q[r]];
-    z[r] = pz[q[r]];
-    w[r] = mass[q[r]];
   }
 #pragma unroll
   for (int r = 0; r < kPer; ++r) {
     const int l = r * 256 + tid;
     float t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (REC) {
-      if (key[r] < sentinel) corner_terms(make_float4(x[r], y[r], z[r], w[r]), t);
-    } else if (key[r] < sentinel) {
-      // the particle's offsets in its cell, recomputed from its coordinates exactly as its
-      // key was (a live key means all three axes are in range)
-      int ix, iy, iz;
-      float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-      (void)pm::cic_axis(x[r], dx, n, ix, fx);
-      (void)pm::cic_axis(y[r], dx, n, iy, fy);
-      (void)pm::cic_axis(z[r], dx, n, iz, fz);
-      corner_terms(make_float4(fx, fy, fz, w[r] * inv_vol), t);
-    }
+    if (key[r] < sentinel) corner_terms(v[r], t);
     keys_l[l + 1] = key[r];
     float4* dst = terms4 + ((l / kChunk) * kTermStride + (l % kChunk) * 8) / 4;
     dst[0] = make_float4(t[0], t[1], t[2], t[3]);
@@ -957,9 +989,11 @@ __global__ void __launch_bounds__(256) reset_listed_kernel(int32_t* __restrict__
                                                            uint8_t* __restrict__ bricks,
                                                            const int32_t* __restrict__ list,
                                                            const uint32_t* __restrict__ count,
-                                                           uint32_t* __restrict__ big_count) {
+                                                           uint32_t* __restrict__ big_count,
+                                                           OrderSample order) {
   const int nb = (n + kBrick - 1) / kBrick;
   if (blockIdx.x == 0 && threadIdx.x == 0) *big_count = 0u;
+  if (order.ordered && blockIdx.x == 0 && threadIdx.x < 64) sample_order(order, n);
   const int64_t m = n + 1;
   constexpr int kSpan = kBrick + 1;  // cells ex in [8bi, 8bi+8]
   const uint32_t cnt = *count;
@@ -979,12 +1013,15 @@ __global__ void __launch_bounds__(256) reset_listed_kernel(int32_t* __restrict__
   }
 }
 
-// map = -1 for every extended cell, bricks = 0, no big cells listed yet.
+// map = -1 for every extended cell, bricks = 0, no big cells listed yet. (Both resets also take
+// the sample of the particles' order: a launch of its own would cost more than the sample.)
 __global__ void __launch_bounds__(256) reset_map_kernel(int32_t* __restrict__ map, int64_t cells,
                                                         uint8_t* __restrict__ bricks,
                                                         int64_t nbricks,
-                                                        uint32_t* __restrict__ big_count) {
+                                                        uint32_t* __restrict__ big_count, int n,
+                                                        OrderSample order) {
   const int64_t i = pm::xcd_block() * blockDim.x + threadIdx.x;
+  if (order.ordered && blockIdx.x == 0 && threadIdx.x < 64) sample_order(order, n);
   if (i < cells) map[i] = -1;
   if (i < nbricks) bricks[i] = 0;
   if (i == 0) *big_count = 0u;
@@ -1086,6 +1123,7 @@ struct pm_deposit_plan {
   // records of the key pass for the piece pass (null in the no-allocation path, whose scratch
   // holds no more; deposits with given keys gather from the particle arrays)
   float4* rec = nullptr;
+  int* ordered = nullptr;       // device: whether the sampled particles lie in cell order
   bool timing = false;
   hipEvent_t ev[5] = {};
   float last_ms[4] = {0, 0, 0, 0};
@@ -1101,7 +1139,7 @@ void free_plan(pm_deposit_plan* p) {
   if (!p) return;
   void* bufs[] = {p->keys[0], p->keys[1], p->vals[0], p->vals[1], p->hist, p->digit,
                   p->sums, p->head, p->tail, p->tail_slot, p->head_end, p->mid_pieces, p->bricks, p->brick_list, p->brick_count, p->map, p->big,
-                  p->big_count, p->big_off, p->rec, p->acc64, p->maxbits};
+                  p->big_count, p->big_off, p->rec, p->ordered, p->acc64, p->maxbits};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (auto& e : p->ev)
@@ -1184,6 +1222,7 @@ pm_status pm_deposit_plan_create(int32_t n, int64_t cap, pm_deposit_plan** out) 
     return alloc(&ptr, count, what);
   });
   if (st == PM_OK) st = alloc(&p->rec, cap, "hipMalloc records");
+  if (st == PM_OK) st = alloc(&p->ordered, 1, "hipMalloc order flag");
   if (st != PM_OK) {
     free_plan(p);
     return st;
@@ -1298,6 +1337,12 @@ pm::depbrick::SortBuffers sort_buffers(pm_deposit_plan* p) {
   return sb;
 }
 
+// From this many particles on the device decides whether the key pass leaves records. Smaller
+// sets are served by the caches in any order, and the shorter piece pass pays alone (in cell
+// order, us with / without: 10,000 on 32^3 58 / 65, 100,000 on 64^3 77 / 77, 300,000 on 128^3
+// 84 / 85, 1M 102 / 100).
+constexpr int64_t kSampleMin = int64_t{1} << 19;
+
 // bin_always: a PM_DEPOSIT_BRICKED deposit bins the particles again (pm_deposit_cic) rather
 // than reusing the last binning (pm_deposit_cic_step without PM_STEP_BIN).
 pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, const float* pz,
@@ -1335,14 +1380,18 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
   const bool timing = plan->timing;
   if (timing) PM_TRY_HIP(hipEventRecord(plan->ev[0], stream));
 
+  // the key pass leaves records; large sets only where the device finds them out of cell order
+  const bool records = plan->rec && !keys_in;
+  const OrderSample sample{px, py, pz, np, dx, plan->sentinel,
+                           records && np >= kSampleMin ? plan->ordered : nullptr};
   {
     PM_TIMED("deposit.fill_map", 4.0 * cells, stream);
     if (plan->map_clean) {
       reset_listed_kernel<<<kPersistentBlocks, pm::kBlock, 0, stream>>>(
-          plan->map, n, plan->bricks, plan->brick_list, plan->brick_count, plan->big_count);
+          plan->map, n, plan->bricks, plan->brick_list, plan->brick_count, plan->big_count, sample);
     } else {
       reset_map_kernel<<<pm::blocks_for(cells), pm::kBlock, 0, stream>>>(
-          plan->map, cells, plan->bricks, nbricks_of(n), plan->big_count);
+          plan->map, cells, plan->bricks, nbricks_of(n), plan->big_count, n, sample);
     }
     PM_CHECK_LAUNCH("reset_map_kernel");
     plan->map_clean = true;  // holds again once this deposit's marks are written
@@ -1369,13 +1418,15 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
   // 1. keys
   const float inv_vol = 1.0f / ((dx * dx) * dx);
   if (!keys_in) {
-    PM_TIMED("deposit.key", 16.0 * np, stream);
-    if (plan->rec)
+    PM_TIMED("deposit.key", (records ? 36.0 : 16.0) * np, stream);
+    if (records)
       key_kernel<true><<<pm::blocks_for(np), pm::kBlock, 0, stream>>>(
-          px, py, pz, mass, inv_vol, np, n, dx, plan->sentinel, plan->keys[0], keys_out, plan->rec);
+          px, py, pz, mass, inv_vol, np, n, dx, plan->sentinel, plan->keys[0], keys_out, plan->rec,
+          sample.ordered);
     else
       key_kernel<false><<<pm::blocks_for(np), pm::kBlock, 0, stream>>>(
-          px, py, pz, mass, inv_vol, np, n, dx, plan->sentinel, plan->keys[0], keys_out, nullptr);
+          px, py, pz, mass, inv_vol, np, n, dx, plan->sentinel, plan->keys[0], keys_out, nullptr,
+          nullptr);
     PM_CHECK_LAUNCH("key_kernel");
   } else if (keys_out) {
     PM_TRY_HIP(hipMemcpyAsync(keys_out, keys_in, sizeof(uint32_t) * np,
@@ -1406,14 +1457,14 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
     PM_TIMED("deposit.piece", 24.0 * np, stream);
     const unsigned piece_blocks = static_cast<unsigned>((np + kPiecePos - 1) / kPiecePos);
     const pm::FastDiv m1 = pm::make_fast_div(static_cast<uint32_t>(n) + 1u);
-    if (plan->rec && !keys_in)
+    if (records)
       piece_kernel<true><<<piece_blocks, 256, 0, stream>>>(
-          skey, sidx, px, py, pz, mass, plan->rec, dx, inv_vol, np, plan->sentinel, chunks,
-          plan->sums, plan->map, plan->head, plan->tail, plan->tail_slot, plan->head_end, n,
+          skey, sidx, px, py, pz, mass, plan->rec, sample.ordered, dx, inv_vol, np, plan->sentinel,
+          chunks, plan->sums, plan->map, plan->head, plan->tail, plan->tail_slot, plan->head_end, n,
           plan->bricks, m1);
     else
       piece_kernel<false><<<piece_blocks, 256, 0, stream>>>(
-          skey, sidx, px, py, pz, mass, nullptr, dx, inv_vol, np, plan->sentinel, chunks,
+          skey, sidx, px, py, pz, mass, nullptr, nullptr, dx, inv_vol, np, plan->sentinel, chunks,
           plan->sums, plan->map, plan->head, plan->tail, plan->tail_slot, plan->head_end, n,
           plan->bricks, m1);
     PM_CHECK_LAUNCH("piece_kernel");
