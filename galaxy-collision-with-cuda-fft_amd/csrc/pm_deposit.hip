@@ -1120,10 +1120,12 @@ struct pm_deposit_plan {
   BigCell* big = nullptr;
   uint32_t* big_count = nullptr;
   int64_t* big_off = nullptr;   // batch offsets of the listed big cells (chunks + 1)
-  // records of the key pass for the piece pass (null in the no-allocation path, whose scratch
-  // holds no more; deposits with given keys gather from the particle arrays)
+  // records of the key pass for the piece pass (16 bytes per particle, taken by the first
+  // sorted deposit without given keys; null where those were refused and in the no-allocation
+  // path: the piece pass then gathers from the particle arrays)
   float4* rec = nullptr;
-  int* ordered = nullptr;       // device: whether the sampled particles lie in cell order
+  int* ordered = nullptr;       // after rec: whether the sampled particles lie in cell order
+  bool rec_asked = false;       // an allocation was tried (or must not be)
   bool timing = false;
   hipEvent_t ev[5] = {};
   float last_ms[4] = {0, 0, 0, 0};
@@ -1139,7 +1141,7 @@ void free_plan(pm_deposit_plan* p) {
   if (!p) return;
   void* bufs[] = {p->keys[0], p->keys[1], p->vals[0], p->vals[1], p->hist, p->digit,
                   p->sums, p->head, p->tail, p->tail_slot, p->head_end, p->mid_pieces, p->bricks, p->brick_list, p->brick_count, p->map, p->big,
-                  p->big_count, p->big_off, p->rec, p->ordered, p->acc64, p->maxbits};
+                  p->big_count, p->big_off, p->rec, p->acc64, p->maxbits};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   for (auto& e : p->ev)
@@ -1218,11 +1220,9 @@ pm_status pm_deposit_plan_create(int32_t n, int64_t cap, pm_deposit_plan** out) 
   // room for small tiles too (the no-allocation scratch keeps to the large ones)
   p->hist_cap = std::max(p->hist_cap,
                          pm::radix::small_hist_words(std::min(cap, pm::radix::kSmallSort)));
-  pm_status st = for_each_buffer(p, [](auto*& ptr, int64_t count, const char* what) {
+  const pm_status st = for_each_buffer(p, [](auto*& ptr, int64_t count, const char* what) {
     return alloc(&ptr, count, what);
   });
-  if (st == PM_OK) st = alloc(&p->rec, cap, "hipMalloc records");
-  if (st == PM_OK) st = alloc(&p->ordered, 1, "hipMalloc order flag");
   if (st != PM_OK) {
     free_plan(p);
     return st;
@@ -1337,6 +1337,36 @@ pm::depbrick::SortBuffers sort_buffers(pm_deposit_plan* p) {
   return sb;
 }
 
+// Allocates the plan's records, once, unless `stream` is being captured (nothing is allocated
+// then; a later deposit may) or they would take more than a quarter of the free memory: they
+// only save time, and must not be what a set near the device's limit fails on. Without them the
+// deposit gathers.
+void want_records(pm_deposit_plan* p, hipStream_t stream) {
+  if (p->rec_asked) return;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return;
+  }
+  p->rec_asked = true;
+  // another thread may be capturing in global mode, which forbids allocations elsewhere too
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  const size_t bytes = sizeof(float4) * (static_cast<size_t>(p->cap) + 1);
+  size_t free_bytes = 0, total = 0;
+  void* ptr = nullptr;
+  if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && bytes <= free_bytes / 4 &&
+      hipMalloc(&ptr, bytes) == hipSuccess) {
+    p->rec = static_cast<float4*>(ptr);
+    p->ordered = reinterpret_cast<int*>(p->rec + p->cap);
+  }
+  (void)hipGetLastError();  // a refusal is no error of the deposit's
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
 // From this many particles on the device decides whether the key pass leaves records. Smaller
 // sets are served by the caches in any order, and the shorter piece pass pays alone (in cell
 // order, us with / without: 10,000 on 32^3 58 / 65, 100,000 on 64^3 77 / 77, 300,000 on 128^3
@@ -1381,6 +1411,7 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
   if (timing) PM_TRY_HIP(hipEventRecord(plan->ev[0], stream));
 
   // the key pass leaves records; large sets only where the device finds them out of cell order
+  if (!keys_in && np > 0) want_records(plan, stream);
   const bool records = plan->rec && !keys_in;
   const OrderSample sample{px, py, pz, np, dx, plan->sentinel,
                            records && np >= kSampleMin ? plan->ordered : nullptr};
@@ -1418,6 +1449,7 @@ pm_status deposit_cic(pm_deposit_plan* plan, const float* px, const float* py, c
   // 1. keys
   const float inv_vol = 1.0f / ((dx * dx) * dx);
   if (!keys_in) {
+    // (16 with records too where the device finds the particles in cell order)
     PM_TIMED("deposit.key", (records ? 36.0 : 16.0) * np, stream);
     if (records)
       key_kernel<true><<<pm::blocks_for(np), pm::kBlock, 0, stream>>>(
@@ -1601,6 +1633,7 @@ pm_status pm_deposit_cic_noalloc(int32_t n, const float* px, const float* py, co
   PM_REQUIRE(np >= 0 && np < (int64_t(1) << 31),
              "pm_deposit_cic_noalloc: particle count must be in [0, 2^31)");
   pm_deposit_plan plan;  // host bookkeeping only; every buffer lies in the scratch array
+  plan.rec_asked = true;
   init_plan_shape(&plan, n, np > 0 ? np : 1);
   const int64_t need = carved_bytes(&plan);
   if (need > PM_DEPOSIT_NOALLOC_SCRATCH_BYTES) {

@@ -46,7 +46,10 @@ int32_t pm_abi_version(void);
  * ---------------------------------------------------------------------------------- */
 typedef struct pm_deposit_plan pm_deposit_plan;
 
-/* Scratch for grids of `grid_size` nodes per axis and up to `max_particles` particles. */
+/* Scratch for grids of `grid_size` nodes per axis and up to `max_particles` particles. The
+ * first sorted-mode deposit without given keys outside a stream capture adds 16 bytes per
+ * particle to it where they are at most a quarter of the free memory (only its time depends on
+ * them). */
 pm_status pm_deposit_plan_create(int32_t grid_size, int64_t max_particles,
                                  pm_deposit_plan** out);
 pm_status pm_deposit_plan_destroy(pm_deposit_plan* plan);

@@ -412,3 +412,53 @@ def test_key_pass_of_ordered_particles_writes_no_records(device):
             best = min(best, plan.last_timing()["key"])
         key_ms.append(best)
     assert key_ms[0] < 0.8 * key_ms[1], key_ms
+
+
+def test_records_are_allocated_when_a_deposit_writes_them(device):
+    """The records' 16 bytes a particle are taken by the first sorted deposit without given keys:
+    not by a plan's creation, a bricked deposit, a deposit with given keys or one under capture."""
+    announce("records allocated by need")
+    from galaxy_collision_amd.deposit import DepositPlan
+
+    n, np_, dx = 32, 1 << 24, 0.5
+    pos, mass = _cell_order(np_, n, dx, device)
+    o = torch.randperm(np_, device=device)
+    x, y, z = (pos[o, a].contiguous() for a in range(3))
+    del pos, o
+    rho = torch.empty((n,) * 3, device=device)
+    keys = torch.empty(np_, dtype=torch.int32, device=device)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    first = used()
+    plan = DepositPlan(n, np_)
+    base = used()
+    # sort and reduction scratch take about 55.3 bytes a particle
+    assert base - first < 60 * np_ + (64 << 20)
+    g = torch.cuda.CUDAGraph()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            plan.deposit(x, y, z, mass, np_, dx, rho, keys)
+    torch.cuda.current_stream().wait_stream(side)
+    outs = []
+    for _ in range(3):
+        rho.fill_(-7.0)
+        g.replay()
+        outs.append(rho.clone())
+    plan.deposit_keyed(x, y, z, mass, np_, dx, rho, keys)
+    ref = rho.clone()
+    assert all(torch.equal(v, ref) for v in outs)
+    torch.cuda.synchronize()
+    assert used() - base < 8 * np_  # captured and keyed: none
+    plan.set_mode("bricked")
+    plan.deposit(x, y, z, mass, np_, dx, rho)
+    plan.set_mode("sorted")
+    mid = used()
+    plan.deposit(x, y, z, mass, np_, dx, rho)
+    assert torch.equal(rho, ref)
+    assert 16 * np_ <= used() - mid < 17 * np_ + (64 << 20)
