@@ -390,15 +390,16 @@ __global__ void __launch_bounds__(256) gather_kernel(
   az[p] = a2;
 }
 
-// Whether the particles lie scattered in memory, from 256 pairs of neighbours spread over the
+// Whether the particles lie scattered in memory, from 64 pairs of neighbours spread over the
 // arrays: in cell order most pairs lie within two cells of each other in x and y, in random
-// order hardly any do. Every workgroup of a launch finds the same answer.
+// order hardly any do. Every wave of a launch finds the same answer by itself (256 pairs and a
+// barrier in 2048 workgroups made the launch cost 3 to 5 us where nothing is interleaved).
 __device__ __forceinline__ bool scattered(const float* __restrict__ px, const float* __restrict__ py,
                                           int64_t np, float dx) {
-  const int64_t p = (np - 1) * static_cast<int64_t>(threadIdx.x) / 256;
+  const int64_t p = (np - 1) * static_cast<int64_t>(threadIdx.x & 63u) / 64;
   const float reach = 2.0f * dx;
   const bool near = fabsf(px[p + 1] - px[p]) <= reach && fabsf(py[p + 1] - py[p]) <= reach;
-  return __syncthreads_count(near) < 128;
+  return __popcll(__ballot(near)) < 32;
 }
 
 // (gx, gy, gz, 0) per node from the three component arrays when the particles are scattered,
@@ -575,9 +576,13 @@ namespace {
 
 // Interleaving the field pays when scattered particles outnumber what the L2 caches serve and
 // are many enough for its 28 bytes a node (random order, us without / with: 300,000 on 128^3
-// 23 / 25, 900,000 on 192^3 80 / 68, 2.1M on 256^3 204 / 181).
+// 23 / 25, 900,000 on 192^3 80 / 68, 2.1M on 256^3 204 / 181). Particles in cell order pay for
+// the launch that finds them so (us without / with: 600,000 on 128^3 8.0 / 10.1, 3M on 192^3
+// 26.9 / 27.5) until the gather's own time covers it (5M on 224^3 40.7 / 39.2, 10M 91.7 / 81.8).
+// 1024 workgroups: 512 end 0.3 us earlier there, but scattered particles gather 122 us after
+// them against 118 (3M); 2048 take 0.5 us longer and gain nothing.
 constexpr int64_t kInterleaveMin = int64_t{1} << 19;
-constexpr unsigned kInterleaveBlocks = 2048;
+constexpr unsigned kInterleaveBlocks = 1024;
 bool interleave_pays(int64_t np, int32_t n) {
   return np >= kInterleaveMin && np >= static_cast<int64_t>(n) * n * n / 8;
 }

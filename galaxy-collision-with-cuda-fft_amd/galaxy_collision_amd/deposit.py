@@ -19,6 +19,7 @@ All arguments are device fields/tensors; work is enqueued on torch's current str
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 
 import torch
@@ -179,16 +180,22 @@ def potential_to_accel(phi, ax_g, ay_g, az_g, dx: float = 1.0) -> None:
              nat.ptr(as_tensor(az_g)), n, float(dx), nat.stream())
 
 
+@functools.lru_cache(maxsize=64)
+def _gather_work_bytes(n_particles: int, grid_size: int) -> int:
+    """Workspace of one gather (a function of the sizes alone)."""
+    size = ctypes.c_int64()
+    nat.call("pm_gather_work_bytes", n_particles, grid_size, ctypes.byref(size))
+    return size.value
+
+
 def gather_acceleration(parts, ax_g, ay_g, az_g, acc_x, acc_y, acc_z, dx: float = 1.0) -> None:
     """CIC-interpolate the node acceleration field to the particles."""
     n = _grid_n(ax_g)
     work = None
     if parts.n >= 1 << 19:  # fewer never need workspace
-        size = ctypes.c_int64()
-        nat.call("pm_gather_work_bytes", int(parts.n), n, ctypes.byref(size))
-        if size.value:  # from torch's allocator, so that it belongs to this call's stream
-            work = torch.empty(size.value // 4, dtype=torch.float32,
-                               device=as_tensor(ax_g).device)
+        size = _gather_work_bytes(int(parts.n), n)
+        if size:  # from torch's allocator, so that it belongs to this call's stream
+            work = torch.empty(size // 4, dtype=torch.float32, device=as_tensor(ax_g).device)
     nat.call("pm_gather_work", nat.ptr(as_tensor(parts.pos_x)), nat.ptr(as_tensor(parts.pos_y)),
              nat.ptr(as_tensor(parts.pos_z)), nat.ptr(as_tensor(ax_g)), nat.ptr(as_tensor(ay_g)),
              nat.ptr(as_tensor(az_g)), nat.ptr(as_tensor(acc_x)), nat.ptr(as_tensor(acc_y)),
