@@ -195,7 +195,10 @@ def gather_acceleration(parts, ax_g, ay_g, az_g, acc_x, acc_y, acc_z, dx: float 
     if parts.n >= 1 << 19:  # fewer never need workspace
         size = _gather_work_bytes(int(parts.n), n)
         if size:  # from torch's allocator, so that it belongs to this call's stream
-            work = torch.empty(size // 4, dtype=torch.float32, device=as_tensor(ax_g).device)
+            try:
+                work = torch.empty(size // 4, dtype=torch.float32, device=as_tensor(ax_g).device)
+            except torch.OutOfMemoryError:
+                pass  # 16 bytes a node that only save time: gather without them
     nat.call("pm_gather_work", nat.ptr(as_tensor(parts.pos_x)), nat.ptr(as_tensor(parts.pos_y)),
              nat.ptr(as_tensor(parts.pos_z)), nat.ptr(as_tensor(ax_g)), nat.ptr(as_tensor(ay_g)),
              nat.ptr(as_tensor(az_g)), nat.ptr(as_tensor(acc_x)), nat.ptr(as_tensor(acc_y)),
