@@ -43,10 +43,14 @@ def scatter_density(parts, img, extent, axes=(0, 1)) -> tuple[float, float]:
     pa, pb = as_tensor(getattr(parts, _AXIS[a])), as_tensor(getattr(parts, _AXIS[b]))
     m = as_tensor(parts.mass)
     # from torch's allocator, so that it belongs to this call's stream
-    work = torch.empty(_work_words(int(parts.n), bins), dtype=torch.int64, device=t.device)
-    nat.call("pm_project_mass_work", nat.ptr(pa), nat.ptr(pb), nat.ptr(m), int(parts.n),
-             lo_a, lo_b, binw_a, binw_b, bins, nat.ptr(t), nat.ptr(work, torch.int64),
-             nat.stream())
+    entry = "pm_project_mass_work"
+    try:
+        work = torch.empty(_work_words(int(parts.n), bins), dtype=torch.int64, device=t.device)
+    except torch.OutOfMemoryError:  # the image's sums alone, and no room for records
+        entry = "pm_project_mass"
+        work = torch.empty(_work_words(0, bins), dtype=torch.int64, device=t.device)
+    nat.call(entry, nat.ptr(pa), nat.ptr(pb), nat.ptr(m), int(parts.n), lo_a, lo_b, binw_a, binw_b,
+             bins, nat.ptr(t), nat.ptr(work, torch.int64), nat.stream())
     return binw_a, binw_b
 
 
