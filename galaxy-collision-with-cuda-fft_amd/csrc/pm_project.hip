@@ -370,10 +370,14 @@ TiledLayout tiled_layout(int64_t n, int bins) {
 // smaller; the tiled path costs 40-90 us up to a million particles, more of it the more tiles
 // a chunk touches. Measured on the collision's disks (direct / tiled, us): 65,536 particles on
 // 128 bins 60 / 42; 200,000 on 512 53 / 53, on 1024 28 / 83; 1,000,000 on 1024 154 / 74;
-// 10,000,002 on 512 3447 / 119 in cell order, 1763 / 133 in random order. kMaxTiles bounds
-// the bins.
+// 10,000,002 on 512 3447 / 119 in cell order, 1763 / 133 in random order. Its launches and
+// passes over short counts cost 18 to 35 us however few the particles, which small images reach
+// only with more particles a bin (direct / tiled, us): 1,000 on 1 bin 19 / 19, 3,000 43 / 28;
+// 6,144 on 4 bins 30 / 32, 10,000 44 / 34; 6,144 on 16 bins 23 / 32, 10,000 33 / 34; 40,000 on
+// 100 37 / 36. kMaxTiles bounds the bins.
 bool use_tiled(int64_t n, int bins) {
-  return n >= int64_t{384} * bins && (bins + kTileSide - 1) / kTileSide <= 16;
+  const int64_t least = std::max<int64_t>(int64_t{384} * bins, std::min(2048 * bins, 10240));
+  return n >= least && (bins + kTileSide - 1) / kTileSide <= 16;
 }
 
 pm_status check_project(const char* who, const float* pos_a, const float* pos_b,

@@ -62,6 +62,26 @@ def test_tiled_projection_matches_integers(device, n, bins, order):
     assert_bitwise(img.cpu().numpy(), _reference(pos, mass, (0.0, side, 0.0, side), bins), "image")
 
 
+@pytest.mark.parametrize("n,bins", [(2048, 1), (8192, 4), (10240, 16), (10240, 26), (384 * 27, 27)])
+def test_tiled_projection_of_few_bins(device, n, bins):
+    """The first tiled sizes of small images: the image of the direct path, and of integers."""
+    test_tiled_projection_matches_integers(device, n, bins, "random")
+    test_tiled_projection_matches_integers(device, n - 1, bins, "random")
+
+
+def test_tiled_projection_rule_at_few_bins(device):
+    """Images of few bins are tiled only from the particles on that pay for the extra launches."""
+    import ctypes
+
+    from galaxy_collision_amd import _native as nat
+
+    size = ctypes.c_int64()
+    for n, bins in ((400, 1), (2047, 1), (3000, 4), (8191, 4), (6144, 16), (10239, 16),
+                    (10239, 26), (384 * 27 - 1, 27)):
+        nat.call("pm_project_work_bytes", n, bins, ctypes.byref(size))
+        assert size.value == (bins * bins + 1) * 8, (n, bins)
+
+
 def test_tiled_projection_workspace_rule(device):
     """The workspace the tiled path asks for stays bounded by its slab of records."""
     import ctypes
