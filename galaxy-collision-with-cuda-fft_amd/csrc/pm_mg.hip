@@ -1721,7 +1721,7 @@ struct pm_mg {
   bool solved = false;
   // warm-start state (allocated on the first pm_mg_solve_warm)
   float* hist = nullptr;      // phi of the previous warm solve (the time history)
-  float* cand = nullptr;      // extrapolated guess of the current solve
+  float* cand = nullptr;      // extrapolated guess of the current solve (training pairs only)
   bool hist_valid = false;
   // carried guess (EXTRAPOLATE without pairs, MIXED): the next solve's guess
   // 2*phi_t - phi_(t-1), written by the updates of the solve before (no extrapolation pass)
@@ -2584,7 +2584,8 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
     }
   }
   const int64_t n0 = mg->lv[0].nodes();
-  if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->f0), sizeof(float) * n0)) ||
+  if ((d.mode == PM_MG_PLAIN &&
+       (st = dalloc(mg, reinterpret_cast<void**>(&mg->f0), sizeof(float) * n0))) ||
       (st = dalloc(mg, reinterpret_cast<void**>(&mg->partials),
                    sizeof(double) * pm::kRedBlocks * pm::kRedMaxQ)) ||
       (st = dalloc(mg, reinterpret_cast<void**>(&mg->red), sizeof(double) * pm::kRedMaxQ)) ||
@@ -2730,12 +2731,12 @@ pm_status pm_mg_solve_warm(pm_mg* mg, const float* rho, float* phi, pm_mg_warm* 
                "pm_mg_solve_warm: network resolution must equal grid_size / pool");
     PM_REQUIRE(w->fallback_ratio > 0.0, "pm_mg_solve_warm: fallback_ratio must be positive");
   }
-  // buffers: time history always; the network grid only when used
-  if (!mg->hist) {
-    if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->hist), sizeof(float) * nodes)) ||
-        (st = dalloc(mg, reinterpret_cast<void**>(&mg->cand), sizeof(float) * nodes)))
-      return st;
-  }
+  // buffers: time history always; the guess and the network grid only when used
+  if (!mg->hist && (st = dalloc(mg, reinterpret_cast<void**>(&mg->hist), sizeof(float) * nodes)))
+    return st;
+  if (w->pair_target && !mg->cand &&
+      (st = dalloc(mg, reinterpret_cast<void**>(&mg->cand), sizeof(float) * nodes)))
+    return st;
   if (want_net_grid && !mg->r32) {
     if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->r32), sizeof(float) * nodes)) ||
         (st = dalloc(mg, reinterpret_cast<void**>(&mg->e0), sizeof(float) * nodes)))

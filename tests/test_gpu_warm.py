@@ -351,3 +351,39 @@ def test_network_correction_and_its_judge(device, n, pool, split):
     assert rec["resid_before"] == pytest.approx(float(pooled(r).pow(2).sum().sqrt()), rel=1e-3)
     after = pooled(r - lap(full)).pow(2).sum().sqrt()
     assert rec["resid_after"] == pytest.approx(float(after), rel=1e-3)
+
+
+def test_solver_memory_follows_its_use(device):
+    """MIXED solves keep no copy of f = 4 pi G rho (the defect and the network scale rho), and the
+    extrapolated guess is kept for training pairs only. Device memory of a 256^3 solver in arrays
+    of n^3 floats: the correction and the defect twice (the split ones the same size), the
+    residual, coarse levels of 1/8 with at most eight arrays each: 6.3; warm solves add the history
+    and the carried guess, then pairs the guess, the network grid being small."""
+    announce("solver memory n=256")
+    from galaxy_collision_amd import _native as nat
+    from galaxy_collision_amd.solver.multigrid import MixedPrecisionMultigridSolver
+
+    n = 256
+    rho = torch.rand((n,) * 3, device=device)
+    phi = torch.zeros((n,) * 3, device=device)
+    pairs = (torch.empty(((n // 4) ** 3, 8), dtype=torch.bfloat16, device=device),
+             torch.empty((n // 4) ** 3, device=device))
+
+    def arrays():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return (total - free) / (4 * n ** 3)
+
+    torch.empty(1, device=device)
+    at = [arrays()]
+    s = MixedPrecisionMultigridSolver(n, dx=0.1, grav_constant=1.0, n_cycles=1, pool=4)
+    at.append(arrays())
+    for _ in range(2):
+        s.solve_warm(rho, phi, nat.PM_WARM_EXTRAPOLATE)
+    at.append(arrays())
+    for _ in range(2):
+        s.solve_warm(rho, phi, nat.PM_WARM_EXTRAPOLATE, *pairs)
+    at.append(arrays())
+    grown = [b - a for a, b in zip(at, at[1:])]
+    print(f"arrays: {grown}", flush=True)
+    assert grown[0] < 6.3 and grown[1] < 2.3 and grown[2] < 1.3
