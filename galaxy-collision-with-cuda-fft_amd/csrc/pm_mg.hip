@@ -1668,7 +1668,7 @@ struct Level {
   float* phi = nullptr;  // level 0: the solve's phi (caller's in PLAIN, e0 in MIXED)
   float* rhs = nullptr;  // level 0: 4*pi*G*rho (PLAIN) or the float32 defect (MIXED)
   float* res = nullptr;
-  float* tmp = nullptr;  // ping-pong partner of phi for the fused sweep (large levels only)
+  float* tmp = nullptr;  // partner of phi for one-launch sweeps and legs (coarse levels)
   float* es = nullptr;   // coarse levels swept in split layout: phi and rhs (zero faces and pads)
   float* rs = nullptr;
   int hs = 0;            // their row length
@@ -1744,8 +1744,9 @@ struct pm_mg {
   std::vector<CycleGraph> graphs;
   hipStream_t capture = nullptr;
   bool use_graphs = true;
-  // MIXED: the finest level's correction and defect in colour-split layout (allocated when
-  // the hierarchy has a coarser level below the finest and pre/post sweeps are >= 1)
+  // the finest level in colour-split layout: MIXED's correction and defect (allocated when the
+  // hierarchy has a coarser level below the finest and pre/post sweeps are >= 1), or PLAIN's phi
+  // and right-hand side (e0s where it fits, r32s in lv[0].res)
   float* e0s = nullptr;
   float* r32s = nullptr;
   int hn = 0;
@@ -1769,6 +1770,30 @@ pm_status dalloc(pm_mg* mg, void** p, size_t bytes) {
   if (e != hipSuccess) return pm::hip_fail("hipMalloc (multigrid)", e);
   mg->owned.push_back(*p);
   return PM_OK;
+}
+
+// Two arrays of `bytes` that only save time: false (and both null) where they do not fit or would
+// take more than a quarter of the free memory, so that a size near the device's limit keeps
+// the room it had for the rest of the run.
+bool dalloc_spare(pm_mg* mg, float** a, float** b, size_t bytes) {
+  size_t free_bytes = 0, total = 0;
+  void* p[2] = {nullptr, nullptr};
+  const size_t need = b ? 2 * bytes : bytes;
+  bool ok = hipMemGetInfo(&free_bytes, &total) == hipSuccess && need <= free_bytes / 4;
+  for (int q = 0; ok && q < (b ? 2 : 1); ++q) ok = hipMalloc(&p[q], bytes) == hipSuccess;
+  if (!ok) {
+    for (void* v : p)
+      if (v) (void)hipFree(v);
+    (void)hipGetLastError();  // a refusal is no error
+    return false;
+  }
+  *a = static_cast<float*>(p[0]);
+  mg->owned.push_back(p[0]);
+  if (b) {
+    *b = static_cast<float*>(p[1]);
+    mg->owned.push_back(p[1]);
+  }
+  return true;
 }
 
 void destroy(pm_mg* mg) {
@@ -2633,32 +2658,28 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
     }
   }
   if (d.mode == PM_MG_PLAIN && d.grid_size % 8 == 0 && d.grid_size >= kPlainSplitMin &&
-      mg->lv.size() > 1 && mg->bottom_from != 0 && d.post_sweeps >= 1) {
+      mg->lv.size() > 1 && mg->bottom_from != 0 && d.post_sweeps >= 1 &&
+      dalloc_spare(mg, &mg->e0s, nullptr, sizeof(float) * n0)) {
+    // rows of whole quads: a split array has the natural size. The split cycle has no use for
+    // the natural residual, so its right-hand side lies there.
     mg->hn = d.grid_size / 2;
-    if ((st = dalloc(mg, reinterpret_cast<void**>(&mg->e0s), sizeof(float) * n0)) ||
-        (st = dalloc(mg, reinterpret_cast<void**>(&mg->r32s), sizeof(float) * n0))) {
-      destroy(mg);
-      return st;
-    }
+    mg->r32s = mg->lv[0].res;
   }
   // coarse levels below a split one, down to the sizes that one launch per leg or sweep serves
   if (mg->e0s && d.pre_sweeps >= 1 && d.post_sweeps >= 1) {
     for (size_t l = 1; l + 1 < mg->lv.size(); ++l) {
       Level& L = mg->lv[l];
       if (L.n <= kLegMax || (mg->bottom_from >= 0 && static_cast<int>(l) >= mg->bottom_from)) break;
-      L.hs = split_row(L.n);
-      const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(L.n) * L.n * L.hs;
-      for (float** q : {&L.es, &L.rs}) {
-        if ((st = dalloc(mg, reinterpret_cast<void**>(q), bytes))) {
-          destroy(mg);
-          return st;
-        }
-        hipError_t ze = hipMemset(*q, 0, bytes);
-        if (ze == hipSuccess) ze = hipDeviceSynchronize();
-        if (ze != hipSuccess) {
-          destroy(mg);
-          return pm::hip_fail("hipMemset (multigrid split levels)", ze);
-        }
+      const int hs = split_row(L.n);
+      const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(L.n) * L.n * hs;
+      if (!dalloc_spare(mg, &L.es, &L.rs, bytes)) break;
+      L.hs = hs;
+      hipError_t ze = hipMemset(L.es, 0, bytes);
+      if (ze == hipSuccess) ze = hipMemset(L.rs, 0, bytes);
+      if (ze == hipSuccess) ze = hipDeviceSynchronize();
+      if (ze != hipSuccess) {
+        destroy(mg);
+        return pm::hip_fail("hipMemset (multigrid split levels)", ze);
       }
     }
   }

@@ -465,3 +465,26 @@ def test_split_levels_equal_natural_levels(device, kind, n, sweeps):
         out.append(phi)
     assert bool(torch.isfinite(out[0]).all())
     assert torch.equal(out[0], out[1])
+
+
+def test_plain_solver_memory(device):
+    """The split layout adds one array of n^3 floats to a PLAIN solver (its right-hand side lies in
+    the natural residual's place) and two to each split coarse level, of 1/8 and 1/64: with
+    f and the residual at the finest level and at most four natural arrays at each coarse one,
+    2 + 4/7 + 1 + 2 * 9/64 = 3.86 arrays; bound 4."""
+    announce("plain solver memory n=256")
+    from galaxy_collision_amd.solver.multigrid import MultigridPoissonSolver
+
+    n = 256
+
+    def arrays():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return (total - free) / (4 * n ** 3)
+
+    MultigridPoissonSolver(8, dx=0.1, grav_constant=1.0)  # what the first one of a process adds
+    before = arrays()
+    s = MultigridPoissonSolver(n, dx=0.1, grav_constant=1.0)
+    grown = arrays() - before
+    print(f"arrays: {grown}", flush=True)
+    assert s is not None and grown < 4.0
