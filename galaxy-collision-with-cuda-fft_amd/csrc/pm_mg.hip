@@ -2558,47 +2558,43 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
   if (mg->d.min_cycles < 1) mg->d.min_cycles = 1;
   const std::vector<int> sizes = level_sizes(d.grid_size, d.mode);
   pm_status st = PM_OK;
+  // (cleared on the null stream; the synchronization at the end is the only one)
+  pm::TimingPause no_timers;
+  auto clear = [](float* p, size_t bytes) {
+    return fill(p, static_cast<int64_t>(bytes / sizeof(float)), 0.0f, nullptr);
+  };
   for (size_t l = 0; l < sizes.size(); ++l) {
     Level L;
     L.n = sizes[l];
     L.h = static_cast<double>(d.dx) * static_cast<double>(int64_t(1) << l);
     L.h2 = static_cast<float>(L.h * L.h);
     L.inv_h2 = static_cast<float>(1.0 / (L.h * L.h));
-    const size_t bytes = sizeof(float) * static_cast<size_t>(L.nodes());
-    if (l > 0) {
-      if ((st = dalloc(mg, reinterpret_cast<void**>(&L.phi), bytes)) ||
-          (st = dalloc(mg, reinterpret_cast<void**>(&L.rhs), bytes))) {
-        destroy(mg);
-        return st;
-      }
+    // one allocation a level; coarse ones are cleared, for their faces are zero for good (legs
+    // and split levels write interior nodes only)
+    const bool inner = l + 1 < sizes.size();
+    float** arrays[4] = {l > 0 ? &L.phi : nullptr, l > 0 ? &L.rhs : nullptr,
+                         inner ? &L.res : nullptr, nullptr};
+    if (L.n >= kSweepMin || (l > 0 && inner && L.n <= std::max(kSmallSweepMax, kLegMax)))
+      arrays[3] = &L.tmp;
+    const size_t bytes = (sizeof(float) * static_cast<size_t>(L.nodes()) + 255) / 256 * 256;
+    size_t at = 0;
+    for (float** q : arrays) at += q ? bytes : 0;
+    void* block = nullptr;
+    if (at && (st = dalloc(mg, &block, at))) {
+      destroy(mg);
+      return st;
     }
-    if (l + 1 < sizes.size()) {
-      if ((st = dalloc(mg, reinterpret_cast<void**>(&L.res), bytes))) {
-        destroy(mg);
-        return st;
-      }
+    if (at && l > 0 && (st = clear(static_cast<float*>(block), at))) {
+      destroy(mg);
+      return st;
     }
-    if (L.n >= kSweepMin ||
-        (l > 0 && l + 1 < sizes.size() && L.n <= std::max(kSmallSweepMax, kLegMax))) {
-      if ((st = dalloc(mg, reinterpret_cast<void**>(&L.tmp), bytes))) {
-        destroy(mg);
-        return st;
-      }
-    }
-    // faces below the finest level are zero for good; the legs write interior nodes only
-    for (float* q : {L.phi, L.rhs, L.tmp}) {
-      const hipError_t ze = l > 0 && q ? hipMemset(q, 0, bytes) : hipSuccess;
-      if (ze != hipSuccess) {
-        destroy(mg);
-        return pm::hip_fail("hipMemset (multigrid levels)", ze);
-      }
+    at = 0;
+    for (float** q : arrays) {
+      if (!q) continue;
+      *q = reinterpret_cast<float*>(static_cast<char*>(block) + at);
+      at += bytes;
     }
     mg->lv.push_back(L);
-  }
-  const hipError_t se = hipDeviceSynchronize();
-  if (se != hipSuccess) {
-    destroy(mg);
-    return pm::hip_fail("hipDeviceSynchronize (multigrid levels)", se);
   }
   // the bottom solver takes over at the first level <= kBottomMax when every level below it
   // is small too and the hierarchy fits its descriptor
@@ -2635,12 +2631,9 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
         return st;
       }
       // faces and pad slots of e0s stay zero for good (no kernel writes them)
-      hipError_t ze = hipMemset(mg->e0s, 0, bytes);
-      if (ze == hipSuccess) ze = hipMemset(mg->r32s, 0, bytes);
-      if (ze == hipSuccess) ze = hipDeviceSynchronize();
-      if (ze != hipSuccess) {
+      if ((st = clear(mg->e0s, bytes)) || (st = clear(mg->r32s, bytes))) {
         destroy(mg);
-        return pm::hip_fail("hipMemset (multigrid split buffers)", ze);
+        return st;
       }
       if (n % 8 == 0) {
         const int64_t quads = static_cast<int64_t>(n) * n * mg->hn / 4;
@@ -2674,12 +2667,9 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
       const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(L.n) * L.n * hs;
       if (!dalloc_spare(mg, &L.es, &L.rs, bytes)) break;
       L.hs = hs;
-      hipError_t ze = hipMemset(L.es, 0, bytes);
-      if (ze == hipSuccess) ze = hipMemset(L.rs, 0, bytes);
-      if (ze == hipSuccess) ze = hipDeviceSynchronize();
-      if (ze != hipSuccess) {
+      if ((st = clear(L.es, bytes)) || (st = clear(L.rs, bytes))) {
         destroy(mg);
-        return pm::hip_fail("hipMemset (multigrid split levels)", ze);
+        return st;
       }
     }
   }
@@ -2687,6 +2677,11 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
   if (he != hipSuccess) {
     destroy(mg);
     return pm::hip_fail("hipHostMalloc", he);
+  }
+  // the arrays cleared above, before any stream takes them
+  if ((he = hipDeviceSynchronize()) != hipSuccess) {
+    destroy(mg);
+    return pm::hip_fail("hipDeviceSynchronize (multigrid)", he);
   }
   *out = mg;
   return PM_OK;
