@@ -799,7 +799,8 @@ FwdPlan fwd_plan(int nvox, int rows, int kpad_, bool allow_split) {
   return p;
 }
 
-// Input channel counts that conv_tile_kernel is built for (192 fill the LDS).
+// Input channel counts that conv_tile_kernel is built for. A tile takes 400 * (2 * channels + 16)
+// bytes of LDS: 108,800 for 128, 83,200 for each half of 192.
 bool tile_fits(int cin) {
   switch (cin) {
     case 8: case 16: case 32: case 48: case 64: case 96: case 128: case 192: return true;
@@ -844,10 +845,15 @@ pm_status fwd_tile(const ConvFwdArgs& a, const char* timer, hipStream_t s) {
   return PM_OK;
 }
 
-int64_t fwd_scratch_floats(int cin, int cout, int r) {
+// Scratch of conv_fwd_kernel's split, whether or not it serves these widths.
+int64_t split_scratch_floats(int cin, int cout, int r) {
   const int64_t nvox = static_cast<int64_t>(r) * r * r;
   const FwdPlan p = fwd_plan(static_cast<int>(nvox), rows_pad(cout), kpad(cin), true);
   return p.ksplit > 1 ? p.ksplit * nvox * rows_pad(cout) : 0;
+}
+
+int64_t fwd_scratch_floats(int cin, int cout, int r) {
+  return tile_fits(cin) ? 0 : split_scratch_floats(cin, cout, r);
 }
 
 pm_status fwd(const uint16_t* xa, int ca, const uint16_t* xb, int cb, int r, int up,
@@ -1076,8 +1082,8 @@ pm_status pm_conv3d_pack_weights(const float* w, int32_t cout, int32_t cin, int3
 
 pm_status pm_conv3d_scratch_size(int32_t cin, int32_t cout, int32_t r, int64_t* floats) {
   PM_REQUIRE(floats && cin >= 1 && cout >= 1 && r >= 1, "pm_conv3d_scratch_size: bad argument");
-  *floats = std::max(pm::conv::fwd_scratch_floats(cin, cout, r),
-                     pm::conv::fwd_scratch_floats(pm::conv::store_channels(cout), cin, r));
+  *floats = std::max(pm::conv::split_scratch_floats(cin, cout, r),
+                     pm::conv::split_scratch_floats(pm::conv::store_channels(cout), cin, r));
   return PM_OK;
 }
 

@@ -63,7 +63,9 @@ struct pm_wsnet {
   float* g = nullptr;             // gradient of an upsampled tensor (coarse)
   float* partial = nullptr;        // backward-weight partial sums
   int64_t partial_floats = 0;
-  float* fscratch = nullptr;       // split-K partial sums of forward / backward-data passes
+  // split-K partial sums of forward / backward-data passes (null where no layer is split: the
+  // LDS-tile kernel serves every width of the packaged network)
+  float* fscratch = nullptr;
   int64_t fscratch_floats = 0;
   float* dout_copy = nullptr;
   bool have_params = false;
@@ -208,7 +210,7 @@ pm_status pm_wsnet_create(const pm_wsnet_desc* desc, pm_wsnet** out) {
                  pm::conv::fwd_scratch_floats(pm::conv::store_channels(l.cout), l.ca + l.cb, l.r)));
   }
   net->partial_floats = part;
-  if ((st = f32(&net->fscratch, std::max<int64_t>(net->fscratch_floats, 4)))) return fail(st);
+  if (net->fscratch_floats > 0 && (st = f32(&net->fscratch, net->fscratch_floats))) return fail(st);
   if ((st = bf(&net->dz, dz_elems)) || (st = f32(&net->g, g_elems)) ||
       (st = f32(&net->partial, part)) || (st = f32(&net->dout_copy, vox(R[0]))))
     return fail(st);

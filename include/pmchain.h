@@ -505,7 +505,10 @@ pm_status pm_conv3d_pack_weights(const float* w, int32_t cout, int32_t cin, int3
                                  uint16_t* packed, hipStream_t stream);
 /* Float32 scratch that lets the two calls below split their reduction over workgroups on
  * small grids (split-K, partial sums folded in a fixed order); without it (scratch null or
- * smaller) they run unsplit. Same result either way up to float32 summation order. */
+ * smaller) they run unsplit. Same result either way up to float32 summation order. An upper
+ * bound: reductions over 8, 16, 32, 48, 64, 96, 128 or 192 channels (the input's in the forward
+ * pass, roundup8(cout) in the backward-data pass) run from an LDS tile, unsplit, and leave the
+ * scratch alone. */
 pm_status pm_conv3d_scratch_size(int32_t cin, int32_t cout, int32_t r, int64_t* floats);
 /* y = act(conv(x) + bias), act 1 = leaky ReLU with negative slope `slope`, 0 = identity.
  * Outputs (either may be null): y bf16 [r^3][roundup8(cout)] (pad channels 0), y32 float32

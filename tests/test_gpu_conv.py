@@ -97,6 +97,8 @@ FWD_CASES = [
 ]
 
 
+# widths that the LDS tile serves: with `split` they are given scratch and leave it alone; the
+# split reduction itself is reached by test_conv_split_reduction_matches_float64
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("r,ca,cb,up,cout,act", FWD_CASES)
 def test_conv_forward_matches_float64(device, r, ca, cb, up, cout, act, split):
@@ -118,7 +120,7 @@ def test_conv_forward_matches_float64(device, r, ca, cb, up, cout, act, split):
     y32 = torch.empty(r ** 3 * cout, dtype=torch.float32, device=device)
     scr, nscr = scratch_for(cin, cout, r, split, device)
     if split:
-        assert nscr > 0, "these small grids split their reduction"
+        assert nscr > 0, "the size query covers a split of these small grids"
     nat.call("pm_conv3d_fwd_bf16", nat.ptr(xa_d, torch.bfloat16), ca,
              nat.ptr(xb_d, torch.bfloat16) if cb else None, cb, r, up,
              nat.ptr(packed, torch.bfloat16), nat.ptr(b_d), cout, act, slope,
@@ -210,6 +212,86 @@ def test_conv_backward_matches_float64_autograd(device, r, ca, cb, up, cout, spl
              nfl.value, nat.stream())
     torch.cuda.synchronize()
     assert rel_l2(dw.cpu().numpy().reshape(cout, cin, 27), 2 * ref_dw) < 1e-5
+
+
+SPLIT_CASES = [
+    # r, ca, cb, up, cout, act: widths without a tile kernel, odd and tiny grids
+    (1, 24, 0, 0, 8, 1),       # one voxel
+    (3, 40, 0, 0, 24, 0),      # 27 voxels, 34 chunks of 32 over splits of unequal length
+    (5, 24, 0, 0, 16, 1),
+    (6, 56, 24, 1, 48, 1),     # 80 = upsampled ++ skip
+    (7, 136, 0, 0, 1, 0),
+    (4, 128, 128, 0, 40, 1),   # the tensor border inside a split
+    (2, 256, 0, 0, 80, 1),
+]
+
+
+@pytest.mark.parametrize("r,ca,cb,up,cout,act", SPLIT_CASES)
+def test_conv_split_reduction_matches_float64(device, r, ca, cb, up, cout, act):
+    """Forward convolutions whose reduction is split over workgroups and folded (conv_fwd_kernel
+    with a range of chunks, conv_epilogue_kernel): the scratch must have been written."""
+    test_conv_forward_matches_float64(device, r, ca, cb, up, cout, act, True)
+    nat = _nat()
+    cin = ca + cb
+    g = torch.Generator().manual_seed(r + cin)
+    ra = r // 2 if up else r
+    xa = bf16_rand((ra ** 3, ca), g).to(device)
+    xb = bf16_rand((r ** 3, cb), g).to(device) if cb else None
+    packed = pack(torch.randn(cout * cin * 27, generator=g).to(device), cout, cin, 0, device)
+    y32 = torch.empty(r ** 3 * cout, dtype=torch.float32, device=device)
+    scr, nscr = scratch_for(cin, cout, r, True, device)
+    scr.fill_(float("nan"))
+    nat.call("pm_conv3d_fwd_bf16", nat.ptr(xa, torch.bfloat16), ca,
+             nat.ptr(xb, torch.bfloat16) if cb else None, cb, r, up,
+             nat.ptr(packed, torch.bfloat16), None, cout, act, 0.1, None, nat.ptr(y32),
+             nat.ptr(scr), nscr, nat.stream())
+    assert bool(torch.isfinite(y32).all())
+    assert bool(torch.isfinite(scr).any()), "the reduction was not split"
+
+
+@pytest.mark.parametrize("r,cin,cout", [(1, 8, 24), (3, 16, 40), (5, 48, 80), (6, 21, 24),
+                                        (4, 64, 250), (7, 1, 136)])
+def test_conv_backward_data_split_matches_float64(device, r, cin, cout):
+    """Backward-data convolutions whose reduction, over roundup8(cout) channels without a tile
+    kernel, is split over workgroups."""
+    announce(f"conv bwd data, split r={r} cin={cin} cout={cout}")
+    nat = _nat()
+    g = torch.Generator().manual_seed(31 + r + cin + cout)
+    w32 = torch.randn(cout, cin, 3, 3, 3, generator=g) / np.sqrt(27 * cin)
+    dz = torch.zeros(r ** 3, store(cout), dtype=torch.bfloat16)
+    dz[:, :cout] = bf16_rand((r ** 3, cout), g)
+    x = torch.zeros(1, cin, r, r, r, dtype=torch.float64, requires_grad=True)
+    y = F.conv3d(x, w32.to(torch.bfloat16).double(), None, padding=1)
+    (y * to_ncdhw(dz[:, :cout].contiguous(), r)).sum().backward()
+    dz_d = dz.reshape(-1).to(device)
+    packed_t = pack(w32.to(device), cout, cin, 1, device)
+    dx = torch.empty(r ** 3 * cin, dtype=torch.float32, device=device)
+    scr, nscr = scratch_for(cin, cout, r, True, device)
+    scr.fill_(float("nan"))
+    nat.call("pm_conv3d_bwd_data_bf16", nat.ptr(dz_d, torch.bfloat16), cout, r,
+             nat.ptr(packed_t, torch.bfloat16), cin, nat.ptr(dx), nat.ptr(scr), nscr,
+             nat.stream())
+    assert rel_l2(dx.cpu().numpy().reshape(r ** 3, cin), to_cl(x.grad).numpy()) < 1e-5
+    assert bool(torch.isfinite(scr).any()), "the reduction was not split"
+
+
+def test_network_takes_no_split_scratch(device):
+    """A network whose widths the LDS tile serves allocates no scratch for split reductions (8 MiB
+    of the 262 that the packaged one took at 64^3; bound half way)."""
+    announce("network memory 64^3")
+    from galaxy_collision_amd.warmstart import WarmStartNet
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return (total - free) / 2 ** 20
+
+    keep = [WarmStartNet(16, seed=1)]
+    before = used()
+    keep.append(WarmStartNet(64, seed=1))
+    took = used() - before
+    print(f"network: {took:.0f} MiB", flush=True)
+    assert took < 258
 
 
 def test_pool_act_upsum_helpers(device):
