@@ -367,16 +367,19 @@ TiledLayout tiled_layout(int64_t n, int bins) {
 }
 
 // The direct path's cost is the queue at the hottest bins, which shortens as the bins get
-// smaller; the tiled path costs 40-90 us up to a million particles, more of it the more tiles
-// a chunk touches. Measured on the collision's disks (direct / tiled, us): 65,536 particles on
-// 128 bins 60 / 42; 200,000 on 512 53 / 53, on 1024 28 / 83; 1,000,000 on 1024 154 / 74;
-// 10,000,002 on 512 3447 / 119 in cell order, 1763 / 133 in random order. Its launches and
-// passes over short counts cost 18 to 35 us however few the particles, which small images reach
-// only with more particles a bin (direct / tiled, us): 1,000 on 1 bin 19 / 19, 3,000 43 / 28;
-// 6,144 on 4 bins 30 / 32, 10,000 44 / 34; 6,144 on 16 bins 23 / 32, 10,000 33 / 34; 40,000 on
-// 100 37 / 36. kMaxTiles bounds the bins.
+// smaller; the tiled path costs 35-70 us up to a million particles, more of it the more tiles a
+// chunk touches. Measured on the collision's disks in random / in cell order (direct, then tiled,
+// us): 98,304 particles on 256 bins 38 / 52, 38 / 40; 196,608 on 512 37 / 47, 43 / 44; 307,200 on
+// 640 48 / 46, 54 / 55, 368,640 57 / 60, 52 / 54; 345,600 on 900 52 / 44, 62 / 65, 518,400 82 / 69,
+// 72 / 70; 491,520 on 1024 59 / 48, 57 / 58, 589,824 64 / 58, 57 / 59; 10,000,002 on 512 1763 /
+// 3447, 133 / 119. So a bin of side wants 384 particles up to 512 bins and 544 above. The launches
+// and the passes over short counts cost 18 to 35 us however few the particles, which small images
+// reach only with more particles a bin (direct / tiled): 1,000 on 1 bin 19 / 19, 3,000 43 / 28;
+// 6,144 on 4 bins 30 / 32, 10,000 44 / 34; 6,144 on 16 bins 23 / 32, 10,000 33 / 34; 40,000 on 100
+// 37 / 36. kMaxTiles bounds the bins.
 bool use_tiled(int64_t n, int bins) {
-  const int64_t least = std::max<int64_t>(int64_t{384} * bins, std::min(2048 * bins, 10240));
+  const int64_t least = std::max<int64_t>(int64_t{bins <= 512 ? 384 : 544} * bins,
+                                          std::min(2048 * bins, 10240));
   return n >= least && (bins + kTileSide - 1) / kTileSide <= 16;
 }
 

@@ -35,7 +35,7 @@ def _reference(pos, mass, extent, bins):
     (384 * 65 + 1, 65, "random"),    # a second tile row of one bin, a last group of few
     (384 * 16, 16, "hot"),           # bins below a tile, every particle in one bin
     (4096 * 97 + 5, 1000, "random"),
-    (4096 * 100, 1024, "sorted"),    # the most tiles, whole waves in one tile
+    (4096 * 100, 1024, "sorted"),    # large images: the direct path below 544 a bin of side
     (8192 * 30, 300, "hot"),         # every chunk adds to one bin
     ((1 << 24) + 4097, 200, "random"),  # more records than the workspace holds at once
 ])
@@ -62,24 +62,34 @@ def test_tiled_projection_matches_integers(device, n, bins, order):
     assert_bitwise(img.cpu().numpy(), _reference(pos, mass, (0.0, side, 0.0, side), bins), "image")
 
 
-@pytest.mark.parametrize("n,bins", [(2048, 1), (8192, 4), (10240, 16), (10240, 26), (384 * 27, 27)])
-def test_tiled_projection_of_few_bins(device, n, bins):
-    """The first tiled sizes of small images: the image of the direct path, and of integers."""
+@pytest.mark.parametrize("n,bins", [(2048, 1), (8192, 4), (10240, 16), (10240, 26), (384 * 27, 27),
+                                    (544 * 513, 513), (4096 * 137 + 5, 1000), (544 * 1024, 1024)])
+def test_tiled_projection_from_its_first_size(device, n, bins):
+    """The first tiled sizes of small and of large images and the last direct ones: the image of
+    integers."""
     test_tiled_projection_matches_integers(device, n, bins, "random")
-    test_tiled_projection_matches_integers(device, n - 1, bins, "random")
+    test_tiled_projection_matches_integers(device, n - 1, bins, "sorted")
 
 
-def test_tiled_projection_rule_at_few_bins(device):
-    """Images of few bins are tiled only from the particles on that pay for the extra launches."""
+def test_tiled_projection_with_the_most_tiles(device):
+    test_tiled_projection_matches_integers(device, 4096 * 140, 1024, "sorted")
+
+
+def test_tiled_projection_rule(device):
+    """Images of few bins, and of more than 512, are tiled only from the particles on that pay for
+    the extra launches and passes."""
     import ctypes
 
     from galaxy_collision_amd import _native as nat
 
     size = ctypes.c_int64()
     for n, bins in ((400, 1), (2047, 1), (3000, 4), (8191, 4), (6144, 16), (10239, 16),
-                    (10239, 26), (384 * 27 - 1, 27)):
+                    (10239, 26), (384 * 27 - 1, 27), (544 * 513 - 1, 513), (345_600, 900),
+                    (544 * 1024 - 1, 1024)):
         nat.call("pm_project_work_bytes", n, bins, ctypes.byref(size))
         assert size.value == (bins * bins + 1) * 8, (n, bins)
+        nat.call("pm_project_work_bytes", 2 * n + 10240, bins, ctypes.byref(size))
+        assert size.value > (bins * bins + 1) * 8, (n, bins)
 
 
 def test_tiled_projection_workspace_rule(device):
