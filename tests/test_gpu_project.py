@@ -133,3 +133,8 @@ def test_projection_without_memory_for_records(device):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(img[0], img[1])
+
+
+def test_tiled_projection_of_a_small_image_in_one_bin(device):
+    """Fewer bins than a tile holds, every particle in one of them."""
+    test_tiled_projection_matches_integers(device, 10240, 16, "hot")
