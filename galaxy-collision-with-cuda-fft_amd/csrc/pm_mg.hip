@@ -2558,10 +2558,16 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
   if (mg->d.min_cycles < 1) mg->d.min_cycles = 1;
   const std::vector<int> sizes = level_sizes(d.grid_size, d.mode);
   pm_status st = PM_OK;
-  // (cleared on the null stream; the synchronization at the end is the only one)
+  // Arrays are cleared on the null stream and waited for before any other stream takes them,
+  // group by group: with one wait at the end the first solve took longer by more than it saved
+  // here (PLAIN, cold 256^3: 7.95 ms in place of 7.55 for 0.15 ms).
   pm::TimingPause no_timers;
   auto clear = [](float* p, size_t bytes) {
     return fill(p, static_cast<int64_t>(bytes / sizeof(float)), 0.0f, nullptr);
+  };
+  auto settle = [] {
+    const hipError_t e = hipDeviceSynchronize();
+    return e == hipSuccess ? PM_OK : pm::hip_fail("hipDeviceSynchronize (multigrid)", e);
   };
   for (size_t l = 0; l < sizes.size(); ++l) {
     Level L;
@@ -2595,6 +2601,10 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
       at += bytes;
     }
     mg->lv.push_back(L);
+  }
+  if ((st = settle())) {
+    destroy(mg);
+    return st;
   }
   // the bottom solver takes over at the first level <= kBottomMax when every level below it
   // is small too and the hierarchy fits its descriptor
@@ -2631,7 +2641,7 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
         return st;
       }
       // faces and pad slots of e0s stay zero for good (no kernel writes them)
-      if ((st = clear(mg->e0s, bytes)) || (st = clear(mg->r32s, bytes))) {
+      if ((st = clear(mg->e0s, bytes)) || (st = clear(mg->r32s, bytes)) || (st = settle())) {
         destroy(mg);
         return st;
       }
@@ -2667,7 +2677,7 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
       const size_t bytes = sizeof(float) * 2 * static_cast<size_t>(L.n) * L.n * hs;
       if (!dalloc_spare(mg, &L.es, &L.rs, bytes)) break;
       L.hs = hs;
-      if ((st = clear(L.es, bytes)) || (st = clear(L.rs, bytes))) {
+      if ((st = clear(L.es, bytes)) || (st = clear(L.rs, bytes)) || (st = settle())) {
         destroy(mg);
         return st;
       }
@@ -2677,11 +2687,6 @@ pm_status pm_mg_create(const pm_mg_desc* desc, pm_mg** out) {
   if (he != hipSuccess) {
     destroy(mg);
     return pm::hip_fail("hipHostMalloc", he);
-  }
-  // the arrays cleared above, before any stream takes them
-  if ((he = hipDeviceSynchronize()) != hipSuccess) {
-    destroy(mg);
-    return pm::hip_fail("hipDeviceSynchronize (multigrid)", he);
   }
   *out = mg;
   return PM_OK;
