@@ -676,8 +676,8 @@ __global__ void __launch_bounds__(256) act_bwd_kernel(const float* __restrict__ 
   dz[idx] = f2bf(g);
 }
 
-// act_bwd_kernel, 8 channels of one voxel per thread (gc and g1_stride multiples of 8, 16-byte
-// aligned arrays): the same values from 16-byte loads, with one voxel index per 8 of them (the
+// act_bwd_kernel, 8 channels of one voxel per thread (gc and dz_c multiples of 8, g1_stride of 4,
+// 16-byte aligned arrays): the same values from 16-byte loads, with one voxel index per 8 of them (the
 // scalar kernel divides in 64 bits for each): 7.3 -> 5.9 us a launch over the layers.
 __global__ void __launch_bounds__(256) act_bwd8_kernel(const float* __restrict__ g1, int g1_stride,
                                                        const float* __restrict__ g2,

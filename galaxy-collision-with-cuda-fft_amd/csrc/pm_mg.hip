@@ -1115,9 +1115,9 @@ __global__ void __launch_bounds__(256) rbs4_first_kernel(float* __restrict__ e,
   *reinterpret_cast<float4*>(e + plane + q.t0) = make_float4(out1[0], out1[1], out1[2], out1[3]);
 }
 
-// residual_s_kernel and restrict_kernel in one pass, 4 positions of both colours (8 consecutive
-// natural nodes) per thread: the fine residual is only ever read by the restriction, so it
-// stays in LDS. A workgroup owns tj coarse rows and marches along i over ti coarse planes:
+// residual_kernel and restrict_kernel in one pass over the split layout, 4 positions of both
+// colours (8 consecutive natural nodes) per thread: the fine residual is only ever read by the
+// restriction, so it stays in LDS. A workgroup owns tj coarse rows and marches along i over ti coarse planes:
 // thread (row, quad) of the 2*tj + 1 fine rows carries e's planes i-1, i, i+1 in registers,
 // writes its residuals of plane i to LDS (even and odd k apart, so that the restriction's
 // stride-2 reads are contiguous), and each thread adds the plane's 9 terms to its (up to
@@ -1267,7 +1267,7 @@ __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4))) 
   }
 }
 
-// prolong_s_kernel, 4 colour-1 positions per thread. The 4 nodes share i, j and the parity
+// prolong_add_kernel on the colour-1 nodes of a split level, 4 positions per thread. The 4 nodes share i, j and the parity
 // of k, so their coarse terms come from the same (di, dj) rows at 4 or 5 consecutive coarse
 // k, loaded once; each node's sum keeps prolong_value's order.
 // Coarse rows (ci0 + a, cj0 + b), a < 2, b < kProlongMaxCj, of a prolongation workgroup,

@@ -387,8 +387,8 @@ pm_status pm_mg_warm_reset(pm_mg* mg);
  *     defect in colour-split layout, with the fill, the colour-0 prolongation and the
  *     update folded into the smoothing passes (needs pre/post sweeps >= 1 and a level below
  *     the finest; otherwise ignored). PLAIN solves on grids of a multiple of 8, from 96 up,
- *     run their cycles on colour-split copies of phi and 4*pi*G*rho (post sweeps >= 1 and a
- *     16-byte aligned phi; otherwise ignored).
+ *     run their cycles on colour-split copies of phi and 4*pi*G*rho (post sweeps >= 1, a
+ *     16-byte aligned phi and room for the copies at creation; otherwise ignored).
  *   PM_MG_OPT_BOTTOM (default 1): the levels of size <= 17 at the bottom of the hierarchy
  *     run their part of each V-cycle in one workgroup with every level in LDS; 0 runs them
  *     with the per-level kernels.

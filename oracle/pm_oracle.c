@@ -1,6 +1,6 @@
 /*
  * pm_oracle.c — CPU restatement of the reference PM force chain. TEST INFRASTRUCTURE ONLY:
- * used by tests/, the smoke check and the CPU-baseline leg of bench.py as the checker;
+ * used by tests/, the smoke check and the CPU-baseline leg of bench.py to check results;
  * never linked into or called by the product library.
  *
  * Two parts:

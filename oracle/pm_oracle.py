@@ -1,7 +1,7 @@
 """CPU oracle for the PM force chain — TEST INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s CPU-baseline leg import this
-module, and only as the checker; the product library never calls it.
+module, and only to check results; the product library never calls it.
 
 It restates the reference (pouyalj/Galaxy-Collision-with-CUDA-FFT, Taichi) in numpy float32
 with the reference's per-element operation order, so single kernels can be compared bit for
